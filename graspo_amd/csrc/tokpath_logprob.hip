@@ -1,9 +1,10 @@
 // tokpath_logprob.hip -- selective log-softmax gather + softmax entropy (gfx950).
 //
-// One workgroup of 256 threads streams one row once (tokpath_stream.h:
-// double-buffered 16-byte loads, 8 vectors per thread per step, non-temporal
-// because nothing re-reads the row).  Each thread keeps an online (m, s, t)
-// state in base-2 units:
+// One workgroup of 256 threads streams one row, or one of the slices a row is
+// cut into when there are few rows, once (tokpath_stream.h: double-buffered
+// 16-byte loads, 8 vectors per thread per step, non-temporal because nothing
+// re-reads the row).  Each thread keeps an online (m, s, t) state in base-2
+// units:
 //   d_i = (x_i - m) * log2(e),  s = sum 2^{d_i},  t = sum 2^{d_i} * d_i
 // so logprob = x_target - m - ln s and entropy = ln s - ln2 * t / s.
 // The row is never written back (no [N, V] log-softmax), so the kernel is
@@ -12,9 +13,14 @@
 // Replaces sequence_log_probs_from_logits (src/graspo/core/graspo_loss.py:19-21)
 // and the logsumexp / logaddexp chunk loop of _selected_token_log_probs_from_hidden
 // (src/graspo/backends/graspoflow/tensor_utils.py:180-186).
+#include <chrono>
+#include <thread>
+
 #include "tokpath_stream.h"
 
 namespace gtp {
+
+int64_t device_cus();  // compute units of the current device
 
 constexpr int kLpBlock = 256;
 constexpr int kLpVecs = 8;  // 16-byte vectors per thread per step
@@ -49,6 +55,24 @@ __device__ __forceinline__ int64_t row_head(const T* row, int64_t V) {
   return up % sizeof(T) ? V : min((int64_t)(up / sizeof(T)), V);
 }
 
+// Block-wide (m, s, t) in wave 0's lanes.  `red` holds one state per wave.
+// The reduction is a kernel's tail once per row or slice: with shuffles and
+// pairwise merges the kernel of 61 rows of 151936 bf16 logits took 13.0 us,
+// this way 11.6.
+__device__ __forceinline__ Lse3 block_lse3_wave0(Lse3 v, float (*red)[3]) {
+  v = wave_lse3_max(v);
+  const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
+  if (lane == 0) {
+    red[wid][0] = v.m;
+    red[wid][1] = v.s;
+    red[wid][2] = v.t;
+  }
+  __syncthreads();
+  const int w = lane & (kLpBlock / kWave - 1);
+  const bool in = lane < kLpBlock / kWave;
+  return wave_lse3_max(in ? Lse3{red[w][0], red[w][1], red[w][2]} : Lse3{kNegInf, 0.0f, 0.0f});
+}
+
 // Calls f(i) for this thread's share of the elements outside
 // [head, head + body).
 template <typename F>
@@ -56,19 +80,58 @@ __device__ __forceinline__ void for_edges(int64_t V, int64_t head, int64_t body,
   for (int64_t j = threadIdx.x; j < V - body; j += kLpBlock) f(j < head ? j : j + body);
 }
 
-// This thread's share of one row [0, V).
-template <typename T>
-__device__ __forceinline__ Lse3 lp_thread_state(const T* __restrict__ row, int64_t V) {
+// Elements [e0, e1) of a row that one workgroup takes: slice k of `slices`,
+// cut at whole vectors of the row's aligned body, the first slice with the
+// row's head and the last one with its end.
+struct Slice {
+  int64_t v0, v1;  // vectors of the aligned body
+  bool first, last;
+};
+template <int E>
+__device__ __forceinline__ Slice slice_of(int64_t nvec, int k, int slices) {
+  // whole groups of 64 vectors, so that a wave's 1 KB loads never straddle two slices
+  const int64_t per = ((nvec + slices - 1) / slices + 63) / 64 * 64;
+  const int64_t v0 = min((int64_t)k * per, nvec);
+  return {v0, min(v0 + per, nvec), k == 0, k == slices - 1};
+}
+
+// Whole vectors of the fold: the entropy's moment is summed as e * d, which
+// is NaN where d = -inf (a logit of -inf, or the padding of the last step);
+// only a block whose moment came out NaN is summed again with d clamped.
+// Clamping every element took one VALU instruction in nine of the fold:
+// bf16 [8192, 151936] 401 us, without it 392.
+template <bool kEntropy, int NG, int E>
+__device__ __forceinline__ void lp_fold_block(Lse3& st, const float (&x)[NG][E]) {
+  if constexpr (!kEntropy) {
+    lse_fold_block<false, NG, E>(st, x);
+  } else {
+    Lse3 nt = st;
+    lse_fold_block_max<true, NG, E, false>(nt, x, block_max_raw<NG, E>(x));
+    if (nt.t != nt.t) {
+      nt = st;
+      lse_fold_block<true, NG, E>(nt, x);
+    }
+    st = nt;
+  }
+}
+
+// This thread's share of slice k of a row [0, V).
+template <typename T, bool kEntropy>
+__device__ __forceinline__ Lse3 lp_thread_state(const T* __restrict__ row, int64_t V, int k,
+                                                int slices) {
   constexpr int E = Vec<T>::kE;
   Lse3 st{kNegInf, 0.0f, 0.0f};
   const int64_t head = row_head(row, V);
   const int64_t nvec = (V - head) / E;
+  const Slice sl = slice_of<E>(nvec, k, slices);
   stream_vectors<T, kLpBlock, kLpVecs, true>(
-      row + head, 0, nvec, [&](float(&x)[kLpVecs][E], int64_t vbase, bool last) {
-        if (last) mask_tail<kLpVecs, E, kLpBlock>(x, vbase, nvec);
-        lse_fold_block<true, kLpVecs, E>(st, x);
+      row + head, sl.v0, sl.v1, [&](float(&x)[kLpVecs][E], int64_t vbase, bool last) {
+        if (last) mask_tail<kLpVecs, E, kLpBlock>(x, vbase, sl.v1);
+        lp_fold_block<kEntropy, kLpVecs, E>(st, x);
       });
-  for_edges(V, head, nvec * E, [&](int64_t i) { lse_fold_one(st, Elem<T>::get(row, i)); });
+  // the row's ends go to its last slice
+  if (sl.last)
+    for_edges(V, head, nvec * E, [&](int64_t i) { lse_fold_one(st, Elem<T>::get(row, i)); });
   return st;
 }
 
@@ -77,24 +140,117 @@ __device__ __forceinline__ int64_t load_target(const void* targets, int t64, int
              : (int64_t)reinterpret_cast<const int32_t*>(targets)[n];
 }
 
-template <typename T>
-__global__ __launch_bounds__(kLpBlock) void logprob_entropy_kernel(
-    const T* __restrict__ logits, int64_t V, int64_t row_stride, const void* __restrict__ targets,
-    int t64, float* __restrict__ out_lp, float* __restrict__ out_H, int32_t* __restrict__ out_status) {
-  __shared__ float red[kLpBlock / kWave][3];
-  const int64_t n = blockIdx.x;
-  const T* row = logits + n * row_stride;
-  const int64_t tgt = load_target(targets, t64, n);
-  const bool tgt_ok = tgt >= 0 && tgt < V;
-  float xt = 0.0f;
-  if (threadIdx.x == 0 && tgt_ok) xt = Elem<T>::get(row, tgt);
-  const Lse3 st = block_lse3<kLpBlock>(lp_thread_state<T>(row, V), red);
-  if (threadIdx.x == 0) {
-    const float ln_s = __builtin_amdgcn_logf(st.s) * kLn2;
-    out_lp[n] = tgt_ok ? raw_logprob(xt, st.m, ln_s) : __builtin_nanf("");
-    if (out_H) out_H[n] = ln_s - kLn2 * st.t / st.s;
-    if (out_status) out_status[n] = tgt_ok ? GTP_ROW_OK : GTP_ROW_BAD_TARGET;
+// B x S rows of logits and their targets, each [B, S] with strides of its
+// own (a shifted view of [B, S + 1, V] logits is read in place).
+struct TokenRows {
+  const void* logits;
+  const void* targets;
+  int64_t V, S, bstride, rstride, tbstride, trstride, ignore;
+  int B, t64, has_ignore;
+  // (sequence, position) of row n; one sequence needs no division
+  __device__ __forceinline__ void at(int64_t n, int64_t& b, int64_t& s) const {
+    b = B > 1 ? (uint32_t)n / (uint32_t)S : 0;
+    s = n - b * S;
   }
+  template <typename T>
+  __device__ __forceinline__ const T* row(int64_t b, int64_t s) const {
+    return reinterpret_cast<const T*>(logits) + b * bstride + s * rstride;
+  }
+  __device__ __forceinline__ int64_t target(int64_t b, int64_t s) const {
+    return load_target(targets, t64, b * tbstride + s * trstride);
+  }
+};
+
+// What a row's state gives: logprob, entropy and status.
+struct TokenOut {
+  float* lp;
+  float* H;
+  int32_t* status;
+  __device__ __forceinline__ void put(int64_t n, const Lse3& st, float xt, bool ok) const {
+    const float ln_s = __builtin_amdgcn_logf(st.s) * kLn2;
+    lp[n] = ok ? raw_logprob(xt, st.m, ln_s) : __builtin_nanf("");
+    if (H) H[n] = ln_s - kLn2 * st.t / st.s;
+    if (status) status[n] = ok ? GTP_ROW_OK : GTP_ROW_BAD_TARGET;
+  }
+};
+
+// Target of a row; an ignored one reads as token 0, which is never bad.
+__device__ __forceinline__ int64_t row_target(const TokenRows& a, int64_t b, int64_t s) {
+  const int64_t t = a.target(b, s);
+  return a.has_ignore && t == a.ignore ? 0 : t;
+}
+
+// Ahead of the rows: clears their arrival counters (n_ctr of them) and tells
+// the host, through one word of its own per workgroup (pinned host memory),
+// whether some target lies outside [0, V).  The host raises on a bad target
+// as soon as this kernel has run (2 us for 61 targets, 5 for 8192), while
+// the rows are still streaming; a reduction of per-row statuses after the
+// rows and its copy to the host held it for the whole kernel and 20 us more
+// (a scoring call of 61 rows 41.6 -> 18.2 us, of 8192 402 -> 382).
+constexpr int kVerdictBlock = 1024;
+__global__ __launch_bounds__(kVerdictBlock) void token_targets_kernel(
+    TokenRows a, int64_t N, uint32_t* __restrict__ ctr, int n_ctr, uint32_t* __restrict__ verdict) {
+  const int64_t first = (int64_t)blockIdx.x * kVerdictBlock + threadIdx.x;
+  const int64_t step = (int64_t)gridDim.x * kVerdictBlock;
+  for (int64_t n = first; n < n_ctr; n += step) ctr[n] = 0;
+  if (!verdict) return;
+  bool bad = false;
+  for (int64_t n = first; n < N; n += step) {
+    int64_t b, s;
+    a.at(n, b, s);
+    const int64_t t = row_target(a, b, s);
+    bad |= t < 0 || t >= a.V;
+  }
+  const int any = __syncthreads_or(bad ? 1 : 0);
+  if (threadIdx.x == 0)
+    __hip_atomic_store(verdict + blockIdx.x, any ? GTP_VERDICT_BAD : GTP_VERDICT_GOOD,
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// slices == 1: one workgroup per row.  Otherwise workgroup (row, slice)
+// publishes its (m, s, t), and the last of the row's workgroups to arrive
+// merges them in order (so the result does not depend on which one that is).
+// A second launch for the merge took 4 us after the 12 of 61 rows.
+template <typename T, bool kEntropy>
+__global__ __launch_bounds__(kLpBlock) void token_logprob_kernel(TokenRows a, TokenOut out,
+                                                                 int slices,
+                                                                 uint32_t* __restrict__ ctr,
+                                                                 float* __restrict__ partial) {
+  __shared__ float red[kLpBlock / kWave][3];
+  const int64_t n = slices > 1 ? blockIdx.x / (uint32_t)slices : blockIdx.x;
+  const int k = (int)(blockIdx.x - n * slices);
+  int64_t b, s;
+  a.at(n, b, s);
+  const T* row = a.row<T>(b, s);
+  const int64_t tgt = row_target(a, b, s);
+  const bool ok = tgt >= 0 && tgt < a.V;
+  float xt = 0.0f;
+  if (threadIdx.x == 0 && ok) xt = Elem<T>::get(row, tgt);
+  Lse3 st = block_lse3_wave0(lp_thread_state<T, kEntropy>(row, a.V, k, slices), red);
+  if (threadIdx.x >= kWave) return;
+  if (slices > 1) {
+    // No release operation: gfx950's agent-scope stores write through to
+    // where the other XCDs' agent-scope loads see them, and vmcnt(0) waits
+    // for their completion before the arrival (a release fence would write
+    // the whole L2 back).
+    float* p = partial + (n * slices + k) * 3;
+    if (threadIdx.x < 3)
+      __hip_atomic_store(p + threadIdx.x, threadIdx.x == 0 ? st.m : threadIdx.x == 1 ? st.s : st.t,
+                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    uint32_t arrived = 0;
+    if (threadIdx.x == 0)
+      arrived = __hip_atomic_fetch_add(ctr + n, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (__builtin_amdgcn_readfirstlane((int)arrived) != slices - 1) return;
+    asm volatile("" ::: "memory");
+    // lane k holds slice k (at most kMaxSlices = 32 of them)
+    p = partial + (n * slices + min((int)threadIdx.x, slices - 1)) * 3;
+    const float m = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const float sm = __hip_atomic_load(p + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const float t = __hip_atomic_load(p + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    st = wave_lse3_max((int)threadIdx.x < slices ? Lse3{m, sm, t} : Lse3{kNegInf, 0.0f, 0.0f});
+  }
+  if (threadIdx.x == 0) out.put(n, st, xt, ok);
 }
 
 // Chunk state layout: [N][4] = (m, s, t_nat, x_target), t_nat = ln2 * t.
@@ -106,7 +262,7 @@ __global__ __launch_bounds__(kLpBlock) void lse_partial_kernel(
   const int64_t n = blockIdx.x;
   const T* row = logits + n * row_stride;
   const int64_t tgt = targets ? load_target(targets, t64, n) - col_offset : -1;
-  Lse3 st = block_lse3<kLpBlock>(lp_thread_state<T>(row, Vc), red);
+  Lse3 st = block_lse3_wave0(lp_thread_state<T, true>(row, Vc, 0, 1), red);
   if (threadIdx.x == 0) {
     float* sp = state + n * 4;
     float xt = __builtin_nanf("");
@@ -199,23 +355,24 @@ struct GradOut<float> {
   __device__ static __forceinline__ void put(float* p, int64_t i, float g) { p[i] = g; }
 };
 
-// One row of g * ([i == t] - p_i), p_i = 2^((x_i - lse) log2 e): the nvec
-// whole vectors from element `head` on go to emit_vec(vector index,
-// gradients), the elements before and after them (every element when nvec ==
-// 0) to emit_one(i, gradient).
+// One slice of a row of g * ([i == t] - p_i), p_i = 2^((x_i - lse) log2 e):
+// its whole vectors (of the nvec from element `head` on) go to
+// emit_vec(vector index, gradients); the last slice also takes the elements
+// before and after the vectors (every element when nvec == 0), one by one to
+// emit_one(i, gradient).
 template <typename T, typename EmitVec, typename EmitOne>
 __device__ __forceinline__ void logprob_backward_row(const T* __restrict__ row, int64_t V,
-                                                     int64_t head, int64_t nvec, int64_t tgt,
-                                                     float g, float lse, EmitVec&& emit_vec,
-                                                     EmitOne&& emit_one) {
+                                                     int64_t head, int64_t nvec, const Slice& sl,
+                                                     int64_t tgt, float g, float lse,
+                                                     EmitVec&& emit_vec, EmitOne&& emit_one) {
   constexpr int E = Vec<T>::kE;
   const float ng = -g;
   stream_vectors<T, kLpBlock, kLpVecs, true>(
-      row + head, 0, nvec, [&](float(&x)[kLpVecs][E], int64_t vbase, bool last) {
+      row + head, sl.v0, sl.v1, [&](float(&x)[kLpVecs][E], int64_t vbase, bool last) {
 #pragma unroll
         for (int k = 0; k < kLpVecs; ++k) {
           const int64_t vi = vbase + (int64_t)k * kLpBlock;
-          if (last && vi >= nvec) continue;
+          if (last && vi >= sl.v1) continue;
           float gr[E];
 #pragma unroll
           for (int j = 0; j < E; ++j)
@@ -230,6 +387,7 @@ __device__ __forceinline__ void logprob_backward_row(const T* __restrict__ row, 
           emit_vec(vi, gr);
         }
       });
+  if (!sl.last) return;
   for_edges(V, head, nvec * E, [&](int64_t i) {
     const float xi = Elem<T>::get(row, i);
     emit_one(i, i == tgt ? -g * expm1f(xi - lse)
@@ -237,35 +395,114 @@ __device__ __forceinline__ void logprob_backward_row(const T* __restrict__ row, 
   });
 }
 
+// Slice k of one row's gradient in the logits' dtype; zeros, without reading
+// the row, where g == 0.
 template <typename T>
-__global__ __launch_bounds__(kLpBlock) void logprob_backward_kernel(
-    const T* __restrict__ logits, int64_t V, int64_t row_stride, int64_t col_offset,
-    const void* __restrict__ targets, int t64, const float* __restrict__ grad_lp,
-    const float* __restrict__ lse_in, T* __restrict__ grad, int64_t grad_stride) {
+__device__ __forceinline__ void logprob_backward_slice(const T* __restrict__ row, int64_t V,
+                                                       int64_t tgt, float g, float lse,
+                                                       T* __restrict__ grow, int k, int slices) {
   constexpr int E = Vec<T>::kE;
-  const int64_t n = blockIdx.x;
-  const T* row = logits + n * row_stride;
-  T* grow = grad + n * grad_stride;
-  const float g = grad_lp[n];
-  const int64_t tgt = load_target(targets, t64, n) - col_offset;  // outside [0, V): no one-hot term
   // a gradient row at the logits row's own alignment (always, when both are
   // contiguous) has its 16-byte boundaries at the same elements
   const bool vec_ok = ((reinterpret_cast<uintptr_t>(row) ^ reinterpret_cast<uintptr_t>(grow)) & 15u) == 0;
   const int64_t head = row_head(row, V);
   const int64_t nvec = vec_ok ? (V - head) / E : 0;
+  const Slice sl = slice_of<E>(nvec, k, slices);
   u32x4* gv = reinterpret_cast<u32x4*>(grow + head);
   if (g == 0.0f) {
     const u32x4 z = {0u, 0u, 0u, 0u};
-    for (int64_t vi = threadIdx.x; vi < nvec; vi += kLpBlock) __builtin_nontemporal_store(z, gv + vi);
-    for_edges(V, head, nvec * E, [&](int64_t i) { GradOut<T>::put(grow, i, 0.0f); });
+    for (int64_t vi = sl.v0 + threadIdx.x; vi < sl.v1; vi += kLpBlock)
+      __builtin_nontemporal_store(z, gv + vi);
+    if (sl.last)
+      for_edges(V, head, nvec * E, [&](int64_t i) { GradOut<T>::put(grow, i, 0.0f); });
     return;
   }
   logprob_backward_row<T>(
-      row, V, head, nvec, tgt, g, lse_in[n],
+      row, V, head, nvec, sl, tgt, g, lse,
       [&](int64_t vi, const float(&gr)[E]) {
         __builtin_nontemporal_store(GradOut<T>::pack(gr), gv + vi);
       },
       [&](int64_t i, float gi) { GradOut<T>::put(grow, i, gi); });
+}
+
+template <typename T>
+__global__ __launch_bounds__(kLpBlock) void logprob_backward_kernel(
+    const T* __restrict__ logits, int64_t V, int64_t row_stride, int64_t col_offset,
+    const void* __restrict__ targets, int t64, const float* __restrict__ grad_lp,
+    const float* __restrict__ lse_in, T* __restrict__ grad, int64_t grad_stride, int slices) {
+  const int64_t n = slices > 1 ? blockIdx.x / (uint32_t)slices : blockIdx.x;
+  const int64_t tgt = load_target(targets, t64, n) - col_offset;  // outside [0, V): no one-hot term
+  logprob_backward_slice<T>(logits + n * row_stride, V, tgt, grad_lp[n], lse_in[n],
+                            grad + n * grad_stride, (int)(blockIdx.x - n * slices), slices);
+}
+
+// The gradient of the logprobs of token_logprob_kernel: each row's lse is
+// x_t - logprob, from one load of its target's logit.  Rows past the first
+// St positions of a sequence, and ignored ones, get zeros.  g is grad_lp per
+// row, or (count given) the gradient of the mean -sum(lp) / count of one
+// scalar.
+template <typename T>
+__global__ __launch_bounds__(kLpBlock) void token_logprob_backward_kernel(
+    TokenRows a, int64_t St, const float* __restrict__ lp, const float* __restrict__ grad_lp,
+    const int64_t* __restrict__ count, T* __restrict__ grad, int64_t gbstride, int64_t grstride,
+    int slices) {
+  const int64_t n = slices > 1 ? blockIdx.x / (uint32_t)slices : blockIdx.x;
+  int64_t b, s;
+  a.at(n, b, s);
+  const T* row = a.row<T>(b, s);
+  float g = 0.0f, lse = 0.0f;
+  int64_t tgt = 0;
+  if (s < St) {
+    tgt = a.target(b, s);
+    if (!(a.has_ignore && tgt == a.ignore)) {
+      const int64_t m = b * St + s;
+      g = count ? -grad_lp[0] / (float)count[0] : grad_lp[m];
+      // a target outside the row has a NaN logprob
+      lse = (tgt >= 0 && tgt < a.V ? Elem<T>::get(row, tgt) : 0.0f) - lp[m];
+    }
+  }
+  logprob_backward_slice<T>(row, a.V, tgt, g, lse, grad + b * gbstride + s * grstride,
+                            (int)(blockIdx.x - n * slices), slices);
+}
+
+// loss = -sum_n lp_n v_n / count, count = sum_n v_n, v_n = 1 unless row n is
+// ignored: F.cross_entropy's mean.  An ignored row is multiplied by 0, so a
+// non-finite logprob of it shows in the loss.  One workgroup: at most some
+// ten thousand rows, 4 bytes of logprob and one target each.
+__global__ __launch_bounds__(1024) void token_mean_kernel(TokenRows a, int64_t N,
+                                                          const float* __restrict__ lp,
+                                                          float* __restrict__ loss,
+                                                          int64_t* __restrict__ count) {
+  __shared__ double rs[1024 / kWave];
+  __shared__ int64_t rc[1024 / kWave];
+  double sum = 0.0;
+  int64_t c = 0;
+  for (int64_t n = threadIdx.x; n < N; n += 1024) {
+    int64_t b, s;
+    a.at(n, b, s);
+    const bool v = !(a.has_ignore && a.target(b, s) == a.ignore);
+    sum += (double)(lp[n] * (v ? 1.0f : 0.0f));
+    c += v;
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    sum += __shfl_xor(sum, o, kWave);
+    c += __shfl_xor(c, o, kWave);
+  }
+  const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
+  if (lane == 0) {
+    rs[wid] = sum;
+    rc[wid] = c;
+  }
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+#pragma unroll
+  for (int w = 1; w < 1024 / kWave; ++w) {
+    sum += rs[w];
+    c += rc[w];
+  }
+  loss[0] = (float)(-sum / (double)c);
+  count[0] = c;
 }
 
 // The same gradient of fp32 logits written as two bf16 arrays, hi = the
@@ -304,7 +541,7 @@ __global__ __launch_bounds__(kLpBlock) void logprob_backward_split_kernel(
     return;
   }
   logprob_backward_row<float>(
-      row, V, head, nvec, tgt, g, lse_in[n],
+      row, V, head, nvec, Slice{0, nvec, true, true}, tgt, g, lse_in[n],
       [&](int64_t vi, const float(&gr)[4]) {
         uint32_t h[4], l[4];
 #pragma unroll
@@ -326,6 +563,198 @@ __global__ __launch_bounds__(kLpBlock) void logprob_backward_split_kernel(
 
 using namespace gtp;
 
+namespace {
+constexpr int kMaxRowSlices = 32;
+
+// Workgroups per row: eight resident workgroups on every CU when there are
+// fewer rows than that, each with about one full step of its stream (32 KB)
+// or more; one per row otherwise.  bf16 [61, 151936] takes 11.6 us in ten
+// slices and 15.7 us in one workgroup per row; from 8 x 256 rows on the chip
+// is full without them ([8192, 151936] runs at 6.5 TB/s of the 7.0 that a
+// read-only pass reaches).
+int row_slices(int dtype, int64_t N, int64_t V) {
+  const int64_t nvec = V / (dtype == GTP_DTYPE_F32 ? 4 : 8);
+  const int64_t step = kLpBlock * kLpVecs;
+  const int64_t want = (8 * device_cus() + N - 1) / N;
+  return (int)max((int64_t)1, min(min(want, (int64_t)kMaxRowSlices), (nvec + step - 1) / step));
+}
+
+// Workspace: the rows' arrival counters, then 3 floats per slice.
+size_t row_slices_bytes(int64_t N, int slices) {
+  return slices > 1 ? (size_t)N * 4 + (size_t)(N * slices) * 12 : 0;
+}
+
+template <typename T>
+void token_logprob_launch(const TokenRows& a, const TokenOut& out, int64_t N, int slices,
+                          uint32_t* ctr, hipStream_t s) {
+  const dim3 grid((unsigned)(N * slices)), block(kLpBlock);
+  float* partial = reinterpret_cast<float*>(ctr + (slices > 1 ? N : 0));
+  if (out.H)
+    launch_timed(token_logprob_kernel<T, true>, grid, block, s, a, out, slices, ctr, partial);
+  else
+    launch_timed(token_logprob_kernel<T, false>, grid, block, s, a, out, slices, ctr, partial);
+}
+
+// GTP_OK and the device form of `r`, with sequences that follow one another
+// at the rows' own stride joined into one.
+int token_rows(const gtp_token_rows* r, TokenRows& a, bool need_targets = true) {
+  if (!r || r->B < 0 || r->S < 0 || r->V <= 0 || (r->S > 1 && r->row_stride < r->V) ||
+      r->batch_stride < 0 || r->row_stride < 0 || r->target_batch_stride < 0 ||
+      r->target_row_stride < 0 || r->dtype < GTP_DTYPE_F32 || r->dtype > GTP_DTYPE_F16)
+    return GTP_ERR_INVALID_ARGUMENT;
+  if (r->B > 0x3FFFFFFll || r->S > 0x3FFFFFFll || (r->B > 0 && r->S > 0x3FFFFFFll / r->B) ||
+      r->V > 0x7FFFFFFFll)
+    return GTP_ERR_UNSUPPORTED;
+  if (r->B > 0 && r->S > 0 && (!r->logits || (need_targets && !r->targets)))
+    return GTP_ERR_INVALID_ARGUMENT;
+  a = TokenRows{r->logits, r->targets, r->V, r->S, r->batch_stride, r->row_stride,
+                r->target_batch_stride, r->target_row_stride, r->ignore_index, (int)r->B,
+                r->targets_int64 ? 1 : 0, r->has_ignore ? 1 : 0};
+  return GTP_OK;
+}
+
+// One sequence of B * S rows where both strides allow it (St: positions with
+// a target; the outputs must be indexed alike).
+void join_rows(TokenRows& a, int64_t St) {
+  if (a.B > 1 && St == a.S && a.bstride == a.S * a.rstride && a.tbstride == a.S * a.trstride) {
+    a.S *= a.B;
+    a.B = 1;
+  }
+}
+}  // namespace
+
+extern "C" size_t gtp_token_logprob_workspace_bytes(int dtype, int64_t N, int64_t V) {
+  if (N <= 0 || V <= 0 || N > 0x3FFFFFFll) return 0;
+  return row_slices_bytes(N, row_slices(dtype, N, V));
+}
+
+extern "C" int gtp_token_logprob_rows(const gtp_token_rows* rows, float* out_logprob,
+                                      float* out_entropy, int32_t* out_status, uint32_t* verdict,
+                                      void* workspace, size_t workspace_bytes, void* stream) {
+  TokenRows a;
+  const int rc = token_rows(rows, a);
+  if (rc != GTP_OK) return rc;
+  const int64_t N = (int64_t)a.B * a.S;
+  if (N > 0 && !out_logprob) return GTP_ERR_INVALID_ARGUMENT;
+  if (N == 0) {
+    for (int i = 0; verdict && i < GTP_VERDICT_WORDS; ++i) verdict[i] = GTP_VERDICT_GOOD;
+    return GTP_OK;
+  }
+  join_rows(a, a.S);
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  int slices = row_slices(rows->dtype, N, a.V);
+  if (!workspace || workspace_bytes < row_slices_bytes(N, slices)) slices = 1;
+  uint32_t* ctr = reinterpret_cast<uint32_t*>(workspace);
+  if (slices > 1 || verdict) {
+    // a few thousand targets per workgroup; the words of those not launched are good
+    const int blocks = (int)min((int64_t)GTP_VERDICT_WORDS, (N + 4095) / 4096);
+    for (int i = blocks; verdict && i < GTP_VERDICT_WORDS; ++i) verdict[i] = GTP_VERDICT_GOOD;
+    hipLaunchKernelGGL(token_targets_kernel, dim3((unsigned)blocks), dim3(kVerdictBlock), 0, s, a,
+                       N, ctr, slices > 1 ? (int)N : 0, verdict);
+  }
+  const TokenOut out{out_logprob, out_entropy, out_status};
+  switch (rows->dtype) {
+    case GTP_DTYPE_BF16:
+      token_logprob_launch<uint16_t>(a, out, N, slices, ctr, s);
+      break;
+    case GTP_DTYPE_F16:
+      token_logprob_launch<_Float16>(a, out, N, slices, ctr, s);
+      break;
+    default:
+      token_logprob_launch<float>(a, out, N, slices, ctr, s);
+  }
+  return hipGetLastError() == hipSuccess ? GTP_OK : GTP_ERR_LAUNCH;
+}
+
+extern "C" int gtp_stream_capturing(void* stream) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(reinterpret_cast<hipStream_t>(stream), &st) == hipSuccess &&
+         st != hipStreamCaptureStatusNone;
+}
+
+extern "C" int gtp_verdict_wait(const uint32_t* verdict, int* bad, void* stream) {
+  if (!verdict || !bad) return GTP_ERR_INVALID_ARGUMENT;
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  auto pending = [&] {
+    for (int i = 0; i < GTP_VERDICT_WORDS; ++i)
+      if (__atomic_load_n(verdict + i, __ATOMIC_RELAXED) == GTP_VERDICT_PENDING) return true;
+    return false;
+  };
+  // The word lands about a microsecond after its kernel; waiting for the
+  // stream instead would wait for the rows too.  The stream's state is
+  // looked at now and then, so that failed work ends the wait.
+  bool done = !pending();
+  for (int round = 0; !done; ++round) {
+    for (int i = 0; i < 2000 && !done; ++i) {
+      __builtin_ia32_pause();
+      done = !pending();
+    }
+    if (done) break;
+    const hipError_t e = hipStreamQuery(s);
+    if (e != hipErrorNotReady) {
+      if (e != hipSuccess || pending()) return GTP_ERR_LAUNCH;
+      break;
+    }
+    // after a few hundred microseconds the stream has other work to do first
+    if (round > 16) std::this_thread::sleep_for(std::chrono::microseconds(20));
+  }
+  *bad = 0;
+  for (int i = 0; i < GTP_VERDICT_WORDS; ++i)
+    *bad |= __atomic_load_n(verdict + i, __ATOMIC_RELAXED) == GTP_VERDICT_BAD;
+  return GTP_OK;
+}
+
+extern "C" int gtp_token_mean_loss(const gtp_token_rows* rows, const float* logprob, float* loss,
+                                   int64_t* count, void* stream) {
+  TokenRows a;
+  const int rc = token_rows(rows, a);
+  if (rc != GTP_OK) return rc;
+  const int64_t N = (int64_t)a.B * a.S;
+  if (!loss || !count || (N > 0 && !logprob)) return GTP_ERR_INVALID_ARGUMENT;
+  join_rows(a, a.S);
+  hipLaunchKernelGGL(token_mean_kernel, dim3(1), dim3(1024), 0,
+                     reinterpret_cast<hipStream_t>(stream), a, N, logprob, loss, count);
+  return hipGetLastError() == hipSuccess ? GTP_OK : GTP_ERR_LAUNCH;
+}
+
+extern "C" int gtp_token_logprob_backward(const gtp_token_rows* rows, int64_t positions,
+                                          const float* logprob, const float* grad,
+                                          const int64_t* mean_count, void* grad_logits,
+                                          int64_t grad_batch_stride, int64_t grad_row_stride,
+                                          void* stream) {
+  TokenRows a;
+  const int rc = token_rows(rows, a, positions != 0);
+  if (rc != GTP_OK) return rc;
+  const int64_t N = (int64_t)a.B * a.S;
+  if (positions < 0 || positions > a.S || grad_batch_stride < 0 ||
+      (a.S > 1 && grad_row_stride < a.V))
+    return GTP_ERR_INVALID_ARGUMENT;
+  if (N == 0) return GTP_OK;
+  if (!grad || !grad_logits || (positions > 0 && !logprob)) return GTP_ERR_INVALID_ARGUMENT;
+  if (grad_batch_stride == a.S * grad_row_stride) join_rows(a, positions);
+  if (a.B == 1) positions = positions == rows->S ? a.S : positions;
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  const int slices = row_slices(rows->dtype, N, a.V);
+  const dim3 grid((unsigned)(N * slices)), block(kLpBlock);
+  switch (rows->dtype) {
+    case GTP_DTYPE_BF16:
+      launch_timed(token_logprob_backward_kernel<uint16_t>, grid, block, s, a, positions, logprob,
+                   grad, mean_count, reinterpret_cast<uint16_t*>(grad_logits), grad_batch_stride,
+                   grad_row_stride, slices);
+      break;
+    case GTP_DTYPE_F16:
+      launch_timed(token_logprob_backward_kernel<_Float16>, grid, block, s, a, positions, logprob,
+                   grad, mean_count, reinterpret_cast<_Float16*>(grad_logits), grad_batch_stride,
+                   grad_row_stride, slices);
+      break;
+    default:
+      launch_timed(token_logprob_backward_kernel<float>, grid, block, s, a, positions, logprob,
+                   grad, mean_count, reinterpret_cast<float*>(grad_logits), grad_batch_stride,
+                   grad_row_stride, slices);
+  }
+  return hipGetLastError() == hipSuccess ? GTP_OK : GTP_ERR_LAUNCH;
+}
+
 extern "C" int gtp_logprob_entropy_rows(const void* logits, int dtype, int64_t N, int64_t V,
                                         int64_t row_stride, const void* targets, int targets_int64,
                                         float* out_logprob, float* out_entropy, int32_t* out_status,
@@ -335,22 +764,17 @@ extern "C" int gtp_logprob_entropy_rows(const void* logits, int dtype, int64_t N
   if (N > 0x7FFFFFFFll) return GTP_ERR_UNSUPPORTED;
   if (N == 0) return GTP_OK;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  const dim3 grid((unsigned)N), block(kLpBlock);
+  const TokenRows a{logits, targets, V, N, 0, row_stride, 0, 1, 0, 1, targets_int64 ? 1 : 0, 0};
+  const TokenOut out{out_logprob, out_entropy, out_status};
   switch (dtype) {
     case GTP_DTYPE_BF16:
-      launch_timed(logprob_entropy_kernel<uint16_t>, grid, block, s,
-                         reinterpret_cast<const uint16_t*>(logits), V, row_stride, targets,
-                         targets_int64, out_logprob, out_entropy, out_status);
+      token_logprob_launch<uint16_t>(a, out, N, 1, nullptr, s);
       break;
     case GTP_DTYPE_F16:
-      launch_timed(logprob_entropy_kernel<_Float16>, grid, block, s,
-                         reinterpret_cast<const _Float16*>(logits), V, row_stride, targets,
-                         targets_int64, out_logprob, out_entropy, out_status);
+      token_logprob_launch<_Float16>(a, out, N, 1, nullptr, s);
       break;
     case GTP_DTYPE_F32:
-      launch_timed(logprob_entropy_kernel<float>, grid, block, s,
-                         reinterpret_cast<const float*>(logits), V, row_stride, targets,
-                         targets_int64, out_logprob, out_entropy, out_status);
+      token_logprob_launch<float>(a, out, N, 1, nullptr, s);
       break;
     default:
       return GTP_ERR_INVALID_ARGUMENT;
@@ -650,25 +1074,26 @@ extern "C" int gtp_logprob_backward_rows(const void* logits, int dtype, int64_t 
   if (N > 0x7FFFFFFFll) return GTP_ERR_UNSUPPORTED;
   if (N == 0) return GTP_OK;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  const dim3 grid((unsigned)N), block(kLpBlock);
+  const int slices = N <= 0x3FFFFFF ? row_slices(dtype, N, V) : 1;
+  const dim3 grid((unsigned)(N * slices)), block(kLpBlock);
   switch (dtype) {
     case GTP_DTYPE_BF16:
       launch_timed(logprob_backward_kernel<uint16_t>, grid, block, s,
                          reinterpret_cast<const uint16_t*>(logits), V, row_stride, col_offset,
                          targets, targets_int64, grad_logprob, lse,
-                         reinterpret_cast<uint16_t*>(grad), grad_stride);
+                         reinterpret_cast<uint16_t*>(grad), grad_stride, slices);
       break;
     case GTP_DTYPE_F16:
       launch_timed(logprob_backward_kernel<_Float16>, grid, block, s,
                          reinterpret_cast<const _Float16*>(logits), V, row_stride, col_offset,
                          targets, targets_int64, grad_logprob, lse,
-                         reinterpret_cast<_Float16*>(grad), grad_stride);
+                         reinterpret_cast<_Float16*>(grad), grad_stride, slices);
       break;
     case GTP_DTYPE_F32:
       launch_timed(logprob_backward_kernel<float>, grid, block, s,
                          reinterpret_cast<const float*>(logits), V, row_stride, col_offset,
                          targets, targets_int64, grad_logprob, lse,
-                         reinterpret_cast<float*>(grad), grad_stride);
+                         reinterpret_cast<float*>(grad), grad_stride, slices);
       break;
     default:
       return GTP_ERR_INVALID_ARGUMENT;

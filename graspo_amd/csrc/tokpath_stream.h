@@ -252,8 +252,9 @@ struct Lse3 {
 };
 
 // Fold a block of raw logits whose maximum is cm (NaN values aside).
-// kEntropy selects whether t is kept.
-template <bool kEntropy, int NG, int E>
+// kEntropy selects whether t is kept; without kClamp a value of -inf (d =
+// -inf, weight 0) makes t NaN.
+template <bool kEntropy, int NG, int E, bool kClamp = true>
 __device__ __forceinline__ void lse_fold_block_max(Lse3& st, const float (&x)[NG][E], float cm) {
   if (cm > st.m) {
     if (st.s > 0.0f) {
@@ -274,10 +275,10 @@ __device__ __forceinline__ void lse_fold_block_max(Lse3& st, const float (&x)[NG
     const float e = __builtin_amdgcn_exp2f(d);
     if (i & 1) {
       s1 += e;
-      if (kEntropy) t1 = __builtin_fmaf(e, fmaxf(d, -256.0f), t1);
+      if (kEntropy) t1 = __builtin_fmaf(e, kClamp ? fmaxf(d, -256.0f) : d, t1);
     } else {
       s0 += e;
-      if (kEntropy) t0 = __builtin_fmaf(e, fmaxf(d, -256.0f), t0);
+      if (kEntropy) t0 = __builtin_fmaf(e, kClamp ? fmaxf(d, -256.0f) : d, t0);
     }
   };
   if (__builtin_fabsf(mb) < 1024.0f) {
@@ -387,6 +388,16 @@ __device__ __forceinline__ void wave_lse2(float& m, float& s) {
   const float sv = m == mw ? s : s * __builtin_amdgcn_exp2f((m - mw) * kLog2e);
   m = mw;
   s = wave_sum_f(sv);
+}
+
+// (m, s, t) merge over a wave the same way: the wave maximum, one rescale per
+// lane, two plain sums.  dl is clamped at -256 so that an empty lane (m =
+// -inf, s = t = 0) adds exactly zero; NaN sums stay NaN.
+__device__ __forceinline__ Lse3 wave_lse3_max(Lse3 v) {
+  const float mw = wave_max_f(v.m);
+  const float dl = v.m == mw ? 0.0f : fmaxf((v.m - mw) * kLog2e, -256.0f);
+  const float f = __builtin_amdgcn_exp2f(dl);
+  return {mw, wave_sum_f(v.s * f), wave_sum_f(f * __builtin_fmaf(dl, v.s, v.t))};
 }
 
 // Block-wide (m, s) of NT threads; every thread gets the result.  `red`

@@ -212,6 +212,110 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> logprob_entropy(const at::Tensor&
   return {lp, H, st};
 }
 
+// [S, V] or [B, S, V] logits with unit column stride and targets of their
+// leading shape, each with its own strides.
+gtp_token_rows token_rows(const at::Tensor& logits, const at::Tensor& targets,
+                          const c10::optional<int64_t>& ignore_index) {
+  TORCH_CHECK(logits.is_cuda(), "graspo_tokpath: logits must be a GPU tensor");
+  const int64_t d = logits.dim();
+  TORCH_CHECK((d == 2 || d == 3) && logits.size(d - 1) > 0 && (logits.size(d - 1) == 1 || logits.stride(d - 1) == 1),
+              "graspo_tokpath: logits must be [S, V] or [B, S, V] with contiguous rows");
+  check_same_device(logits, targets, "targets");
+  TORCH_CHECK((targets.scalar_type() == at::kInt || targets.scalar_type() == at::kLong) &&
+                  targets.dim() == d - 1 && targets.sizes() == logits.sizes().slice(0, d - 1),
+              "graspo_tokpath: targets must be int32/int64 of the logits' leading shape");
+  gtp_token_rows r;
+  r.logits = logits.data_ptr();
+  r.targets = targets.data_ptr();
+  r.dtype = dtype_code(logits);
+  r.targets_int64 = targets.scalar_type() == at::kLong;
+  r.has_ignore = ignore_index.has_value();
+  r.ignore_index = ignore_index.value_or(0);
+  r.B = d == 3 ? logits.size(0) : 1;
+  r.S = logits.size(d - 2);
+  r.V = logits.size(d - 1);
+  r.batch_stride = d == 3 ? logits.stride(0) : 0;
+  r.row_stride = logits.stride(d - 2);
+  r.target_batch_stride = d == 3 ? targets.stride(0) : 0;
+  r.target_row_stride = targets.stride(d - 2);
+  return r;
+}
+
+// (logprob, entropy or an empty tensor, mean loss, counted rows, whether a
+// target lies outside [0, V)).  mean: also -sum(logprob) / count.  Waits for
+// the look at the targets, which runs ahead of the rows, not for the rows.
+std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor, bool> token_logprob(
+    const at::Tensor& logits, const at::Tensor& targets, c10::optional<int64_t> ignore_index,
+    bool entropy, bool mean, int64_t stream) {
+  const gtp_token_rows r = token_rows(logits, targets, ignore_index);
+  void* st = reinterpret_cast<void*>(stream);
+  TORCH_CHECK(!gtp_stream_capturing(st),
+              "graspo_tokpath.token_logprob: waits for the targets, so it cannot be captured");
+  const int64_t N = r.B * r.S;
+  const auto f32 = logits.options().dtype(at::kFloat);
+  at::Tensor lp = at::empty(targets.sizes(), f32);
+  at::Tensor H = at::empty({0}, f32), loss = H, count = H;
+  if (entropy) H = at::empty(targets.sizes(), f32);
+  if (mean) {
+    loss = at::empty({}, f32);
+    count = at::empty({}, f32.dtype(at::kLong));
+  }
+  at::Tensor words = at::empty({GTP_VERDICT_WORDS},
+                               at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+  uint32_t* verdict = reinterpret_cast<uint32_t*>(words.data_ptr<int32_t>());
+  for (int i = 0; i < GTP_VERDICT_WORDS; ++i) verdict[i] = GTP_VERDICT_PENDING;
+  const size_t ws_bytes = gtp_token_logprob_workspace_bytes(r.dtype, N, r.V);
+  at::Tensor ws;
+  if (ws_bytes) ws = at::empty({(int64_t)ws_bytes}, logits.options().dtype(at::kByte));
+  check_rc(gtp_token_logprob_rows(&r, lp.data_ptr<float>(), entropy ? H.data_ptr<float>() : nullptr,
+                                  nullptr, verdict, ws_bytes ? ws.data_ptr() : nullptr, ws_bytes,
+                                  st),
+           "gtp_token_logprob_rows");
+  const int mean_rc = mean ? gtp_token_mean_loss(&r, lp.data_ptr<float>(), loss.data_ptr<float>(),
+                                                 count.data_ptr<int64_t>(), st)
+                           : GTP_OK;
+  // before any other error is raised: the words must outlive the kernel
+  int bad = 0;
+  check_rc(gtp_verdict_wait(verdict, &bad, st), "gtp_verdict_wait");
+  check_rc(mean_rc, "gtp_token_mean_loss");
+  return {lp, H, loss, count, bad != 0};
+}
+
+// The gradient of token_logprob's logprobs by its logits, contiguous, of the
+// logits' shape and dtype.  The first `targets.size(-1)` positions of each
+// sequence have a target; mean_count: `grad` is the gradient of the mean.
+at::Tensor token_logprob_backward(const at::Tensor& logits, const at::Tensor& targets,
+                                  const at::Tensor& logprob, const at::Tensor& grad,
+                                  const c10::optional<at::Tensor>& mean_count,
+                                  c10::optional<int64_t> ignore_index, int64_t stream) {
+  const int64_t d = logits.dim();
+  TORCH_CHECK((d == 2 || d == 3) && targets.dim() == d - 1 &&
+                  targets.size(d - 2) <= logits.size(d - 2),
+              "graspo_tokpath.token_logprob_backward: bad shapes");
+  const int64_t S = logits.size(d - 2), St = targets.size(d - 2);
+  gtp_token_rows r = token_rows(logits.narrow(d - 2, 0, St), targets, ignore_index);
+  r.logits = logits.data_ptr();
+  r.S = S;  // positions St.. have no target: their gradient is zero
+  const bool is_mean = mean_count.has_value();
+  for (const at::Tensor* t : {&logprob, &grad}) {
+    check_same_device(logits, *t, "logprob / grad");
+    TORCH_CHECK(t->scalar_type() == at::kFloat && t->is_contiguous(),
+                "graspo_tokpath.token_logprob_backward: logprob and grad must be contiguous float32");
+  }
+  TORCH_CHECK(logprob.numel() == targets.numel() &&
+                  grad.numel() == (is_mean ? 1 : targets.numel()) &&
+                  (!is_mean || (mean_count->scalar_type() == at::kLong && mean_count->numel() == 1)),
+              "graspo_tokpath.token_logprob_backward: logprob, grad and mean_count must match the "
+              "targets");
+  if (is_mean) check_same_device(logits, *mean_count, "mean_count");
+  at::Tensor out = at::empty(logits.sizes(), logits.options());
+  check_rc(gtp_token_logprob_backward(&r, St, logprob.data_ptr<float>(), grad.data_ptr<float>(),
+                                      is_mean ? mean_count->data_ptr<int64_t>() : nullptr,
+                                      out.data_ptr(), S * r.V, r.V, reinterpret_cast<void*>(stream)),
+           "gtp_token_logprob_backward");
+  return out;
+}
+
 void lse_partial(const at::Tensor& logits, const c10::optional<at::Tensor>& targets,
                  int64_t col_offset, const at::Tensor& state, bool accumulate, int64_t stream) {
   check_rows(logits, "logits");
@@ -574,6 +678,14 @@ TORCH_LIBRARY(graspo_tokpath, m) {
       &sample_route);
   m.def("logprob_entropy(Tensor logits, Tensor targets, int stream) -> (Tensor, Tensor, Tensor)",
         &logprob_entropy);
+  m.def(
+      "token_logprob(Tensor logits, Tensor targets, int? ignore_index, bool entropy, bool mean, "
+      "int stream) -> (Tensor, Tensor, Tensor, Tensor, bool)",
+      &token_logprob);
+  m.def(
+      "token_logprob_backward(Tensor logits, Tensor targets, Tensor logprob, Tensor grad, "
+      "Tensor? mean_count, int? ignore_index, int stream) -> Tensor",
+      &token_logprob_backward);
   m.def(
       "lse_partial(Tensor logits, Tensor? targets, int col_offset, Tensor(a!) state, "
       "bool accumulate, int stream) -> ()",

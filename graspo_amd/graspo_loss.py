@@ -14,39 +14,43 @@ from torch import nn
 from . import ops
 
 
-def _rows_logprob_entropy_status(logits: torch.Tensor, output_ids: torch.Tensor):
-    """(logprob, entropy, status) over the last dim of ``logits`` [..., V];
-    views whose leading dims cannot be flattened without a copy are walked
-    per slice."""
+def _token_rows(logits: torch.Tensor) -> torch.Tensor | None:
+    """``logits`` [..., V] as [N, V], or [B, S, V] where the leading dims
+    cannot be flattened without a copy (a shifted view); None when neither
+    does without one."""
+    try:
+        return logits.view(-1, logits.shape[-1])
+    except RuntimeError:
+        return logits if logits.dim() == 3 else None
+
+
+def _rows_logprob_entropy(logits: torch.Tensor, output_ids: torch.Tensor, entropy: bool = True):
+    """(logprob, entropy) over the last dim of ``logits`` [..., V] (entropy
+    empty unless asked for); a target outside [0, V) raises ``RuntimeError``,
+    as the reference's ``gather`` rejects such an index (one wait for the
+    kernel).  Views whose leading dims fit no [B, S, V] without a copy are
+    walked per slice."""
     V = logits.shape[-1]
     lead = logits.shape[:-1]
     if logits.stride(-1) != 1:
         logits = logits.contiguous()
-    try:
-        rows = logits.view(-1, V)
-    except RuntimeError:
-        rows = None
-    if rows is not None:
-        lp, H, st = ops.logprob_entropy(rows, output_ids.reshape(-1))
-        return lp.view(lead), H.view(lead), st.view(lead)
-    parts = [_rows_logprob_entropy_status(logits[i], output_ids[i])
-             for i in range(logits.shape[0])]
-    return tuple(torch.stack(p) for p in zip(*parts))
-
-
-def _rows_logprob_entropy(logits: torch.Tensor, output_ids: torch.Tensor):
-    """(logprob, entropy); a target outside [0, V) raises ``RuntimeError``, as
-    the reference's ``gather`` rejects such an index (one host
-    synchronisation on the per-row status)."""
-    lp, H, st = _rows_logprob_entropy_status(logits, output_ids)
-    ops.raise_on_bad_status(st.reshape(-1), "sequence_log_probs_from_logits")
-    return lp, H
+    rows = _token_rows(logits)
+    if rows is None:
+        parts = [_rows_logprob_entropy(logits[i], output_ids[i], entropy)
+                 for i in range(logits.shape[0])]
+        return tuple(torch.stack(p) for p in zip(*parts))
+    t = output_ids.reshape(rows.shape[:-1])
+    out = ops.token_logprob(rows, t, entropy=entropy)
+    if out.bad_target:
+        status = torch.where((t < 0) | (t >= V), ops.ROW_BAD_TARGET, ops.ROW_OK)
+        ops.raise_on_bad_status(status.reshape(-1), "sequence_log_probs_from_logits")
+    return out.logprob.view(lead), out.entropy.view(lead) if entropy else out.entropy
 
 
 class _SequenceLogProbs(torch.autograd.Function):
     @staticmethod
     def forward(ctx, logits, output_ids):
-        lp, _ = _rows_logprob_entropy(logits, output_ids)
+        lp, _ = _rows_logprob_entropy(logits, output_ids, entropy=False)
         ctx.save_for_backward(logits, output_ids, lp)
         return lp
 
@@ -54,12 +58,13 @@ class _SequenceLogProbs(torch.autograd.Function):
     def backward(ctx, grad_out):
         logits, output_ids, lp = ctx.saved_tensors
         # d logprob_t / d x = onehot(t) - softmax(x), with softmax from the
-        # saved lse = x_t - logprob_t: one read of the logits, one write
-        V = logits.shape[-1]
-        rows = logits.reshape(-1, V)
-        t = output_ids.reshape(-1).to(torch.int64)
-        lse = rows.gather(1, t.unsqueeze(1)).squeeze(1).float() - lp.reshape(-1)
-        grad = ops.logprob_backward(rows, t, grad_out.reshape(-1), lse)
+        # lse = x_t - logprob_t: one read of the logits, one write
+        if logits.stride(-1) != 1:
+            logits = logits.contiguous()
+        rows = _token_rows(logits)
+        if rows is None:
+            rows = logits.reshape(-1, logits.shape[-1])
+        grad = ops.token_logprob_backward(rows, output_ids.reshape(rows.shape[:-1]), lp, grad_out)
         return grad.view(logits.shape), None
 
 
@@ -68,7 +73,7 @@ def sequence_log_probs_from_logits(logits: torch.Tensor, output_ids: torch.Tenso
     Accepts fp32, bf16 or fp16 logits of shape [..., V]; differentiable."""
     if logits.requires_grad and torch.is_grad_enabled():
         return _SequenceLogProbs.apply(logits, output_ids)
-    lp, _ = _rows_logprob_entropy(logits, output_ids)
+    lp, _ = _rows_logprob_entropy(logits, output_ids, entropy=False)
     return lp
 
 

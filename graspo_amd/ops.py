@@ -2,7 +2,8 @@
 
 Each function validates nothing beyond what the native op checks, enqueues
 the HIP kernels on the caller's current stream and returns device tensors;
-none of them synchronises the host.
+none of them synchronises the host except ``token_logprob``, whose callers
+raise on a bad target.
 """
 
 from __future__ import annotations
@@ -120,6 +121,43 @@ def logprob_entropy(logits: torch.Tensor, targets: torch.Tensor):
     if targets.dtype not in (torch.int32, torch.int64):
         targets = targets.to(torch.int64)
     return ops.logprob_entropy(logits, targets.contiguous(), _stream(logits))
+
+
+def _targets(targets: torch.Tensor) -> torch.Tensor:
+    return targets if targets.dtype in (torch.int32, torch.int64) else targets.to(torch.int64)
+
+
+class TokenLogprob(NamedTuple):
+    logprob: torch.Tensor  # fp32, the targets' shape
+    entropy: torch.Tensor  # fp32, the targets' shape (empty unless asked for)
+    mean_loss: torch.Tensor  # fp32 scalar, -sum(logprob) / count (empty unless asked for)
+    count: torch.Tensor    # int64 scalar, rows in the mean (empty unless asked for)
+    bad_target: bool       # some target that is not ignored lies outside [0, V)
+
+
+def token_logprob(logits: torch.Tensor, targets: torch.Tensor, *, ignore_index: int | None = None,
+                  entropy: bool = False, mean: bool = False) -> TokenLogprob:
+    """log_softmax(logits)[targets] over [S, V] or [B, S, V] ``logits`` (unit
+    column stride, read in place) and ``targets`` of their leading shape, one
+    HBM read.  ``entropy`` adds the rows' softmax entropies, ``mean`` the mean
+    cross-entropy over the targets that are not ``ignore_index`` (an ignored
+    row's logprob is token 0's).  Waits for a look at the targets, which runs
+    ahead of the rows, to say whether one is bad."""
+    return TokenLogprob(*load().token_logprob(logits, _targets(targets), ignore_index, entropy,
+                                              mean, _stream(logits)))
+
+
+def token_logprob_backward(logits: torch.Tensor, targets: torch.Tensor, logprob: torch.Tensor,
+                           grad: torch.Tensor, *, mean_count: torch.Tensor | None = None,
+                           ignore_index: int | None = None) -> torch.Tensor:
+    """The gradient of :func:`token_logprob` by ``logits`` (contiguous, their
+    shape and dtype) from its ``logprob`` and the fp32 ``grad`` per row, or of
+    its mean (``mean_count`` given, ``grad`` the loss's).  ``targets`` may
+    cover only the first positions of each sequence: the rest, and ignored
+    rows, get zeros."""
+    return load().token_logprob_backward(
+        logits, _targets(targets), logprob, grad.to(torch.float32).contiguous(), mean_count,
+        ignore_index, _stream(logits))
 
 
 def logprob_backward(logits: torch.Tensor, targets: torch.Tensor, grad_logprob: torch.Tensor,

@@ -18,34 +18,20 @@ from . import ops
 class _SFTCrossEntropy(torch.autograd.Function):
     @staticmethod
     def forward(ctx, logits, labels, ignore_index):
-        B, S, V = logits.shape
-        tgt = labels[:, 1:]
-        valid = tgt.ne(ignore_index)
-        safe = torch.where(valid, tgt, torch.zeros_like(tgt)).to(torch.int64)
-        lp = torch.empty((B, S - 1), dtype=torch.float32, device=logits.device)
-        bad = torch.zeros((), dtype=torch.bool, device=logits.device)
-        for b in range(B):  # the S - 1 rows of one sequence share one row stride
-            lp_b, _, st_b = ops.logprob_entropy(logits[b, : S - 1], safe[b])
-            lp[b] = lp_b
-            bad |= st_b.ne(ops.ROW_OK).any()
-        if bool(bad):  # F.cross_entropy rejects a label outside [0, V)
+        # positions 0 .. S - 2 against labels 1 .. S - 1, both read in place
+        out = ops.token_logprob(logits[:, :-1], labels[:, 1:], ignore_index=ignore_index,
+                                mean=True)
+        if out.bad_target:  # F.cross_entropy rejects a label outside [0, V)
             raise RuntimeError("sft_cross_entropy_loss: a label is outside [0, vocab_size)")
-        count = valid.sum()
-        loss = -(lp * valid).sum() / count
-        ctx.save_for_backward(logits, safe, valid, lp, count)
-        return loss
+        ctx.save_for_backward(logits, labels, out.logprob, out.count)
+        ctx.ignore_index = ignore_index
+        return out.mean_loss
 
     @staticmethod
     def backward(ctx, grad_loss):
-        logits, safe, valid, lp, count = ctx.saved_tensors
-        B, S, V = logits.shape
-        g = torch.where(valid, -grad_loss.float() / count, torch.zeros_like(lp))
-        grad = torch.empty_like(logits, memory_format=torch.contiguous_format)
-        grad[:, S - 1].zero_()
-        for b in range(B):
-            rows = logits[b, : S - 1]
-            lse = rows.gather(1, safe[b].unsqueeze(1)).squeeze(1).float() - lp[b]
-            ops.logprob_backward(rows, safe[b], g[b], lse, out=grad[b, : S - 1])
+        logits, labels, lp, count = ctx.saved_tensors
+        grad = ops.token_logprob_backward(logits, labels[:, 1:], lp, grad_loss, mean_count=count,
+                                          ignore_index=ctx.ignore_index)
         return grad, None, None
 
 

@@ -232,6 +232,77 @@ int gtp_logprob_entropy_rows(const void* logits, int dtype, int64_t N,
                              void* stream);
 
 /*
+ * The rows of the three entry points below: logits [B, S, V] and targets
+ * [B, S], each with its own strides (elements), so that the shifted rows of
+ * [B, S + 1, V] logits are read in place.  With has_ignore a target equal to
+ * ignore_index is no target (as F.cross_entropy's): its row never has a bad
+ * one, is not counted in the mean and gets no gradient.
+ */
+typedef struct gtp_token_rows {
+  const void* logits;
+  const void* targets;    /* int32 (targets_int64 == 0) or int64 */
+  int64_t B, S, V;
+  int64_t batch_stride, row_stride;
+  int64_t target_batch_stride, target_row_stride;
+  int64_t ignore_index;
+  int dtype, targets_int64, has_ignore;
+} gtp_token_rows;
+
+/*
+ * gtp_token_logprob_rows -- gtp_logprob_entropy_rows over gtp_token_rows,
+ * outputs [B * S] in (sequence, position) order.  An ignored row's logprob is
+ * token 0's.  Few rows are cut into slices for several workgroups each, whose
+ * partial states go through a workspace of gtp_token_logprob_workspace_bytes
+ * (B * S rows) bytes, 16-byte aligned, no contents carried between calls;
+ * without one (or when that is 0) each row is one workgroup's.
+ *
+ * verdict, when given, is GTP_VERDICT_WORDS words of host memory that the
+ * device can write (pinned), each GTP_VERDICT_PENDING before the call: a
+ * small kernel ahead of the rows sets each to GTP_VERDICT_GOOD, or to
+ * GTP_VERDICT_BAD when one of its targets lies outside [0, V).
+ * gtp_verdict_wait waits for the words alone (the rows may still be
+ * streaming), *bad != 0 for a bad target; the words must live until then.
+ * Not under stream capture.
+ *
+ * Replaces sequence_log_probs_from_logits  src/graspo/core/graspo_loss.py:19-21
+ * and the forward of F.cross_entropy in sft_cross_entropy_loss
+ * src/graspo/core/sft_loss.py:12-34 (with gtp_token_mean_loss).
+ */
+#define GTP_VERDICT_WORDS 16
+#define GTP_VERDICT_PENDING 0u
+#define GTP_VERDICT_GOOD 1u
+#define GTP_VERDICT_BAD 2u
+int gtp_token_logprob_rows(const gtp_token_rows* rows, float* out_logprob, float* out_entropy,
+                           int32_t* out_status, uint32_t* verdict, void* workspace,
+                           size_t workspace_bytes, void* stream);
+size_t gtp_token_logprob_workspace_bytes(int dtype, int64_t N, int64_t V);
+int gtp_verdict_wait(const uint32_t* verdict, int* bad, void* stream);
+
+/* gtp_stream_capturing -- nonzero while `stream` is being captured. */
+int gtp_stream_capturing(void* stream);
+
+/* gtp_token_mean_loss -- *loss = -sum logprob / *count over the rows that are
+ * not ignored (NaN when there is none), *count their number. */
+int gtp_token_mean_loss(const gtp_token_rows* rows, const float* logprob, float* loss,
+                        int64_t* count, void* stream);
+
+/*
+ * gtp_token_logprob_backward -- the gradient of gtp_token_logprob_rows'
+ * logprobs with respect to the logits, in the logits' dtype: one read of the
+ * logits and one write of the gradient.  Only the first `positions` rows of
+ * each sequence have a target; the others, and ignored ones, get zeros.
+ *   logprob     [B * positions], the forward's
+ *   grad        [B * positions], dL/dlogprob per row; with mean_count it is
+ *               dL/dloss of gtp_token_mean_loss (one value) and mean_count
+ *               that call's *count
+ *   grad_logits [B, S, V] with its own strides
+ */
+int gtp_token_logprob_backward(const gtp_token_rows* rows, int64_t positions,
+                               const float* logprob, const float* grad,
+                               const int64_t* mean_count, void* grad_logits,
+                               int64_t grad_batch_stride, int64_t grad_row_stride, void* stream);
+
+/*
  * gtp_lse_partial_rows -- fold one vocabulary chunk [col_offset, col_offset+Vc)
  * into a running per-row state (m, s, t, x_target), all fp32:
  *   m = running max, s = sum exp(x - m), t = sum exp(x - m) * (x - m),
