@@ -189,7 +189,8 @@ __device__ __forceinline__ int64_t row_target(const TokenRows& a, int64_t b, int
 // (a scoring call of 61 rows 41.6 -> 18.2 us, of 8192 402 -> 382).
 constexpr int kVerdictBlock = 1024;
 __global__ __launch_bounds__(kVerdictBlock) void token_targets_kernel(
-    TokenRows a, int64_t N, uint32_t* __restrict__ ctr, int n_ctr, uint32_t* __restrict__ verdict) {
+    TokenRows a, int64_t N, uint32_t* __restrict__ ctr, int n_ctr, const uint32_t* flag_a,
+    const uint32_t* flag_b, uint32_t* __restrict__ verdict) {
   const int64_t first = (int64_t)blockIdx.x * kVerdictBlock + threadIdx.x;
   const int64_t step = (int64_t)gridDim.x * kVerdictBlock;
   for (int64_t n = first; n < n_ctr; n += step) ctr[n] = 0;
@@ -202,9 +203,10 @@ __global__ __launch_bounds__(kVerdictBlock) void token_targets_kernel(
     bad |= t < 0 || t >= a.V;
   }
   const int any = __syncthreads_or(bad ? 1 : 0);
-  if (threadIdx.x == 0)
-    __hip_atomic_store(verdict + blockIdx.x, any ? GTP_VERDICT_BAD : GTP_VERDICT_GOOD,
-                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  if (threadIdx.x != 0) return;
+  uint32_t w = GTP_VERDICT_GOOD | (any ? GTP_VERDICT_BAD : 0u);
+  if ((flag_a && *flag_a) || (flag_b && *flag_b)) w |= GTP_VERDICT_FLAGGED;
+  __hip_atomic_store(verdict + blockIdx.x, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // slices == 1: one workgroup per row.  Otherwise workgroup (row, slice)
@@ -584,6 +586,16 @@ size_t row_slices_bytes(int64_t N, int slices) {
   return slices > 1 ? (size_t)N * 4 + (size_t)(N * slices) * 12 : 0;
 }
 
+// The look at the targets: a few thousand per workgroup; the words of
+// workgroups that are not launched are good.
+void targets_launch(const TokenRows& a, int64_t N, uint32_t* ctr, int n_ctr, const uint32_t* flag_a,
+                    const uint32_t* flag_b, uint32_t* verdict, hipStream_t s) {
+  const int blocks = (int)max((int64_t)1, min((int64_t)GTP_VERDICT_WORDS, (N + 4095) / 4096));
+  for (int i = blocks; verdict && i < GTP_VERDICT_WORDS; ++i) verdict[i] = GTP_VERDICT_GOOD;
+  hipLaunchKernelGGL(token_targets_kernel, dim3((unsigned)blocks), dim3(kVerdictBlock), 0, s, a, N,
+                     ctr, n_ctr, flag_a, flag_b, verdict);
+}
+
 template <typename T>
 void token_logprob_launch(const TokenRows& a, const TokenOut& out, int64_t N, int slices,
                           uint32_t* ctr, hipStream_t s) {
@@ -645,13 +657,8 @@ extern "C" int gtp_token_logprob_rows(const gtp_token_rows* rows, float* out_log
   int slices = row_slices(rows->dtype, N, a.V);
   if (!workspace || workspace_bytes < row_slices_bytes(N, slices)) slices = 1;
   uint32_t* ctr = reinterpret_cast<uint32_t*>(workspace);
-  if (slices > 1 || verdict) {
-    // a few thousand targets per workgroup; the words of those not launched are good
-    const int blocks = (int)min((int64_t)GTP_VERDICT_WORDS, (N + 4095) / 4096);
-    for (int i = blocks; verdict && i < GTP_VERDICT_WORDS; ++i) verdict[i] = GTP_VERDICT_GOOD;
-    hipLaunchKernelGGL(token_targets_kernel, dim3((unsigned)blocks), dim3(kVerdictBlock), 0, s, a,
-                       N, ctr, slices > 1 ? (int)N : 0, verdict);
-  }
+  if (slices > 1 || verdict)
+    targets_launch(a, N, ctr, slices > 1 ? (int)N : 0, nullptr, nullptr, verdict, s);
   const TokenOut out{out_logprob, out_entropy, out_status};
   switch (rows->dtype) {
     case GTP_DTYPE_BF16:
@@ -672,8 +679,8 @@ extern "C" int gtp_stream_capturing(void* stream) {
          st != hipStreamCaptureStatusNone;
 }
 
-extern "C" int gtp_verdict_wait(const uint32_t* verdict, int* bad, void* stream) {
-  if (!verdict || !bad) return GTP_ERR_INVALID_ARGUMENT;
+extern "C" int gtp_verdict_wait(const uint32_t* verdict, int* found, void* stream) {
+  if (!verdict || !found) return GTP_ERR_INVALID_ARGUMENT;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   auto pending = [&] {
     for (int i = 0; i < GTP_VERDICT_WORDS; ++i)
@@ -698,11 +705,24 @@ extern "C" int gtp_verdict_wait(const uint32_t* verdict, int* bad, void* stream)
     // after a few hundred microseconds the stream has other work to do first
     if (round > 16) std::this_thread::sleep_for(std::chrono::microseconds(20));
   }
-  *bad = 0;
-  for (int i = 0; i < GTP_VERDICT_WORDS; ++i)
-    *bad |= __atomic_load_n(verdict + i, __ATOMIC_RELAXED) == GTP_VERDICT_BAD;
+  uint32_t all = 0;
+  for (int i = 0; i < GTP_VERDICT_WORDS; ++i) all |= __atomic_load_n(verdict + i, __ATOMIC_RELAXED);
+  *found = (int)(all >> 1);  // without GTP_VERDICT_GOOD
   return GTP_OK;
 }
+
+extern "C" int gtp_targets_verdict(const void* targets, int targets_int64, int64_t N,
+                                   int64_t target_stride, int64_t V, const uint32_t* flag_a,
+                                   const uint32_t* flag_b, uint32_t* verdict, void* stream) {
+  if (N < 0 || V <= 0 || target_stride < 0 || (N > 0 && !targets) || !verdict)
+    return GTP_ERR_INVALID_ARGUMENT;
+  if (N > 0x7FFFFFFFll) return GTP_ERR_UNSUPPORTED;
+  const TokenRows a{nullptr, targets, V, N, 0, 0, 0, target_stride, 0, 1, targets_int64 ? 1 : 0, 0};
+  // at least one workgroup, which looks at the flags
+  targets_launch(a, N, nullptr, 0, flag_a, flag_b, verdict, reinterpret_cast<hipStream_t>(stream));
+  return hipGetLastError() == hipSuccess ? GTP_OK : GTP_ERR_LAUNCH;
+}
+
 
 extern "C" int gtp_token_mean_loss(const gtp_token_rows* rows, const float* logprob, float* loss,
                                    int64_t* count, void* stream) {

@@ -160,6 +160,29 @@ def token_logprob_backward(logits: torch.Tensor, targets: torch.Tensor, logprob:
         ignore_index, _stream(logits))
 
 
+class TargetsVerdict:
+    """A look at ``targets`` [N] (ids outside [0, vocab) are bad) and at up to
+    two int32 device flags, queued on the current stream when this is made;
+    :meth:`wait` waits for it alone, not for work queued after it."""
+
+    def __init__(self, targets: torch.Tensor, vocab: int, *flags: torch.Tensor):
+        a, b = (tuple(flags) + (None, None))[:2]
+        self._stream = _stream(targets)
+        self._words = load().verdict_begin(_targets(targets), int(vocab), a, b, self._stream)
+        self._found = None
+
+    def wait(self) -> tuple[bool, bool]:
+        """(a target is bad, a flag is set)."""
+        if self._found is None:
+            self._found = load().verdict_end(self._words, self._stream)
+        return bool(self._found & 1), bool(self._found & 2)
+
+    def __del__(self):
+        # the kernel writes the words: they outlive it
+        if getattr(self, "_found", None) is None and hasattr(self, "_words"):
+            self.wait()
+
+
 def logprob_backward(logits: torch.Tensor, targets: torch.Tensor, grad_logprob: torch.Tensor,
                      lse: torch.Tensor, col_offset: int = 0,
                      out: torch.Tensor | None = None) -> torch.Tensor:

@@ -258,11 +258,11 @@ typedef struct gtp_token_rows {
  *
  * verdict, when given, is GTP_VERDICT_WORDS words of host memory that the
  * device can write (pinned), each GTP_VERDICT_PENDING before the call: a
- * small kernel ahead of the rows sets each to GTP_VERDICT_GOOD, or to
+ * small kernel ahead of the rows sets each to GTP_VERDICT_GOOD, with
  * GTP_VERDICT_BAD when one of its targets lies outside [0, V).
  * gtp_verdict_wait waits for the words alone (the rows may still be
- * streaming), *bad != 0 for a bad target; the words must live until then.
- * Not under stream capture.
+ * streaming); *found gets 1 for a bad target and 2 for a flag, or 0; the words
+ * must live until then.  Not under stream capture.
  *
  * Replaces sequence_log_probs_from_logits  src/graspo/core/graspo_loss.py:19-21
  * and the forward of F.cross_entropy in sft_cross_entropy_loss
@@ -270,13 +270,25 @@ typedef struct gtp_token_rows {
  */
 #define GTP_VERDICT_WORDS 16
 #define GTP_VERDICT_PENDING 0u
-#define GTP_VERDICT_GOOD 1u
-#define GTP_VERDICT_BAD 2u
+#define GTP_VERDICT_GOOD 1u     /* looked at; plus, when found: */
+#define GTP_VERDICT_BAD 2u      /* a target outside [0, V) */
+#define GTP_VERDICT_FLAGGED 4u  /* a nonzero flag of gtp_targets_verdict */
 int gtp_token_logprob_rows(const gtp_token_rows* rows, float* out_logprob, float* out_entropy,
                            int32_t* out_status, uint32_t* verdict, void* workspace,
                            size_t workspace_bytes, void* stream);
 size_t gtp_token_logprob_workspace_bytes(int dtype, int64_t N, int64_t V);
-int gtp_verdict_wait(const uint32_t* verdict, int* bad, void* stream);
+int gtp_verdict_wait(const uint32_t* verdict, int* found, void* stream);
+
+/*
+ * gtp_targets_verdict -- that kernel alone, over N targets target_stride
+ * elements apart; flag_a and flag_b (device words, may be NULL) are looked at
+ * too, e.g. gtp_f32_to_bf16_exact's *inexact.  Serves the hidden-state path,
+ * whose reference raises on an id outside the vocabulary
+ * (tensor_utils.py:167-186, index_select).
+ */
+int gtp_targets_verdict(const void* targets, int targets_int64, int64_t N, int64_t target_stride,
+                        int64_t V, const uint32_t* flag_a, const uint32_t* flag_b,
+                        uint32_t* verdict, void* stream);
 
 /* gtp_stream_capturing -- nonzero while `stream` is being captured. */
 int gtp_stream_capturing(void* stream);
