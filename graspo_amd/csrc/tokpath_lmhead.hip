@@ -26,20 +26,27 @@
 // vocabulary tiles merge afterwards.
 //
 // Order of work.  The workgroup for (vocabulary group g, token tile j) runs
-// kTilesPerGroup vocabulary tiles in a row (its K loop runs on across the
-// tile boundary), merging each tile into its running state, and writes one
-// partial state per (g, wave half, token).  Workgroup b = g * n_tt + j runs
-// on XCD b mod 8, so with 32 token tiles the 32 workgroups that share an
-// XCD's L2 at a time cover 8 vocabulary groups x 4 token tiles: 12 operand
-// tiles per K step come into that L2 (the fewest for 32 workgroups; a whole
-// vocabulary group per XCD would bring in 33), and the window of 8 groups
-// is read from HBM once (the hidden states stay in the last-level cache).
+// one or two vocabulary tiles in a row (its K loop runs on across the tile
+// boundary), merging each tile into its running state, and writes one
+// partial state per (g, wave half, token).  Workgroup b runs on XCD b mod 8.
+// The 32 workgroups that share an XCD's L2 at a time should cover about 8 x 4
+// operand tiles: 12 then come into that L2 per K step (the fewest for 32
+// workgroups; one token tile with 32 vocabulary groups would bring in 33).
+// So up to 8 token tiles an XCD takes all of them for every 8th vocabulary
+// group, up to 16 half of them for every 4th, and above that b = g * n_tt + j
+// (with 32 token tiles 8 groups x 4 tiles).  In that last order 8 token tiles
+// gave each XCD one token tile: 2048 x 4096 x 151936 took 2.47 ms (and its
+// partial tile's own launch 0.11), this way 2.35 for all of it (7.23 -> 7.02
+// ms of the whole training step).
 // A merge kernel folds the partials and the target logits (one fp32 dot
 // product per token, the reference's own selected_logits) into logprob,
 // entropy and lse.
 #include "tokpath_stream.h"
 
 namespace gtp {
+
+int64_t device_cus();  // compute units of the current device
+
 namespace lmh {
 
 constexpr int kBV = 256;                 // vocabulary rows per tile
@@ -55,7 +62,8 @@ constexpr int kYB = 256 / 32 / kWTn;      // 32-token blocks per wave
 constexpr int kQ = 32 / kWaves;           // 1 KB loads per wave per operand and K step
 constexpr int kChunks = kBK / 8;         // 16-byte chunks per tile row
 constexpr int kStage = kBV * kChunks;    // 16-byte chunks per operand stage (32 KB)
-constexpr int kTilesPerGroup = 2;        // vocabulary tiles per workgroup
+constexpr int kMaxTiles = 2;             // vocabulary tiles per workgroup
+constexpr int kXcds = 8;
 constexpr int kMaxLd = (1 << 22) - 1;    // row strides (elements): 256 rows fit a buffer range
 constexpr int kRsrcWord3 = 0x00020000;   // raw buffer: 32-bit data format, no swizzle
 
@@ -68,6 +76,8 @@ struct Args {
   const uint16_t* h;  // [N, K] bf16, row stride ldh
   int64_t V, N, K, ldw, ldh;
   int n_vfull, n_tt, n_vg;  // full vocabulary tiles, token tiles, groups of full tiles
+  int tiles, tail;          // full tiles per group; whether group n_vg is a partial tile
+  int blocks;               // token-tile blocks an XCD chooses from: 1, 2 or 8
   float4* partial;          // [2 * n_vg + 2][N]: (m, s, t, 0), t in base-2 units
   float* logits;            // [V, N] fp32, vocabulary-major, row stride ldl (kStore only)
   int64_t ldl;
@@ -102,9 +112,29 @@ __device__ __forceinline__ float swap_halves(float v) {
   return __int_as_float(__shfl_xor(__float_as_int(v), 32, kWave));
 }
 
-// kTail = false: the full vocabulary tiles, kTilesPerGroup per workgroup.
-// kTail = true: the last, partial tile (V mod 256 rows), one per token tile,
-// its rows past V masked in the epilogue; its partials follow the groups'.
+// The (vocabulary group, token tile) of workgroup b; false for one past the
+// last (the orders below round up).
+__device__ __forceinline__ bool tile_of(const Args& a, int b, int& vg, int& tt) {
+  if (a.blocks == kXcds) {
+    tt = b % a.n_tt;
+    vg = b / a.n_tt;
+  } else {
+    const int x = b % kXcds, i = b / kXcds;
+    const int width = (a.n_tt + a.blocks - 1) / a.blocks;  // token tiles per block
+    tt = (x % a.blocks) * width + i % width;
+    vg = (i / width) * (kXcds / a.blocks) + x / a.blocks;
+  }
+  return tt < a.n_tt && vg < a.n_vg + a.tail;
+}
+// Workgroups of that order.
+inline int64_t grid_of(int n_vg_all, int n_tt, int blocks) {
+  if (blocks == kXcds) return (int64_t)n_vg_all * n_tt;
+  const int per = kXcds / blocks, width = (n_tt + blocks - 1) / blocks;
+  return (int64_t)kXcds * ((n_vg_all + per - 1) / per) * width;
+}
+
+// The last group is the partial tile (V mod 256 rows) when there is one, its
+// rows past V masked in the epilogue.
 // kStore: the epilogue also writes every logit of the tile to a.logits,
 // vocabulary-major: one non-temporal dword store per value, whose 32 lanes of
 // a lane half hold 32 consecutive tokens of one vocabulary row, so that each
@@ -112,24 +142,14 @@ __device__ __forceinline__ float swap_halves(float v) {
 // past N are not written).  Token-major 16-byte stores (4 rows of a token
 // per lane, 32 bytes per token row per instruction) cost 4.2 ms on top of
 // the 13.5 ms GEMM at 8192 x 4096 x 248320.
+// kTail: the partial tile's instance, whose epilogue masks.  (Both instances
+// of the whole body under one branch: two epilogues behind one tile loop
+// spilled 150-230 registers.)
 template <bool kTail, bool kStore>
-__global__ __launch_bounds__(kThreads, 1) void lm_head_lse_kernel(Args a) {
-  __shared__ __attribute__((aligned(16))) uint4 sA0[kStage], sA1[kStage], sB0[kStage], sB1[kStage];
-
-  // ---- which tiles: token tiles fastest
-  const int b = blockIdx.x;
-  int tt, vg, vt0, ntiles;
-  if constexpr (kTail) {
-    tt = b;
-    vg = a.n_vg;
-    vt0 = a.n_vfull;
-    ntiles = 1;
-  } else {
-    tt = b % a.n_tt;
-    vg = b / a.n_tt;
-    vt0 = vg * kTilesPerGroup;
-    ntiles = min(kTilesPerGroup, a.n_vfull - vt0);
-  }
+__device__ __forceinline__ void lm_head_tiles(const Args& a, int vg, int tt, uint4* sA0, uint4* sA1,
+                                              uint4* sB0, uint4* sB1) {
+  const int vt0 = kTail ? a.n_vfull : vg * a.tiles;
+  const int ntiles = kTail ? 1 : min(a.tiles, a.n_vfull - vt0);
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -254,7 +274,7 @@ __global__ __launch_bounds__(kThreads, 1) void lm_head_lse_kernel(Args a) {
   };
 
   // fold the finished tile into the running state and clear the accumulators;
-  // in the tail kernel rows past V read as -inf.  A lane folds its 64 values
+  // in the partial tile rows past V read as -inf.  A lane folds its 64 values
   // of a token one 16-value MFMA block at a time (online: a block with a new
   // maximum rescales (s, t) by 2^dl), so only 16 accumulators are held in
   // VGPRs at a time; then the two lane halves and the running state merge.
@@ -374,6 +394,17 @@ __global__ __launch_bounds__(kThreads, 1) void lm_head_lse_kernel(Args a) {
   }
 }
 
+template <bool kStore>
+__global__ __launch_bounds__(kThreads, 1) void lm_head_lse_kernel(Args a) {
+  __shared__ __attribute__((aligned(16))) uint4 sA0[kStage], sA1[kStage], sB0[kStage], sB1[kStage];
+  int tt, vg;
+  if (!tile_of(a, blockIdx.x, vg, tt)) return;
+  if (vg == a.n_vg)
+    lm_head_tiles<true, kStore>(a, vg, tt, sA0, sA1, sB0, sB1);
+  else
+    lm_head_tiles<false, kStore>(a, vg, tt, sA0, sA1, sB0, sB1);
+}
+
 // x_t = h_n . w_{t_n} in fp32 (bf16 products are exact), one wave per token.
 __global__ __launch_bounds__(256) void lm_head_target_kernel(const uint16_t* __restrict__ w,
                                                              const uint16_t* __restrict__ h,
@@ -445,7 +476,7 @@ __global__ __launch_bounds__(256) void lm_head_merge_kernel(const float4* __rest
 }
 
 struct Plan {
-  int n_vfull, n_tt, n_vg;
+  int n_vfull, n_tt, n_vg, tiles, blocks;
   bool tail;
   size_t partial_bytes, xt_bytes;
 };
@@ -455,7 +486,19 @@ inline Plan plan(int64_t N, int64_t V) {
   p.n_vfull = (int)(V / kBV);
   p.tail = V % kBV != 0;
   p.n_tt = (int)((N + kBT - 1) / kBT);
-  p.n_vg = (p.n_vfull + kTilesPerGroup - 1) / kTilesPerGroup;
+  // Tiles per workgroup: one workgroup per CU at a time, so a launch takes
+  // rounds x tiles tile times.  Two tiles halve the partial states and the
+  // pipeline fills; one leaves less of the chip idle in the last round
+  // (2048 x 4096 x 151936: 19 tile times against 20, 535 x 2816 x 151936: 7
+  // against 8), and is taken when that saves more than 3%.
+  p.blocks = p.n_tt <= 8 ? 1 : p.n_tt <= 16 ? 2 : kXcds;
+  const int64_t cus = device_cus();
+  auto rounds = [&](int t) {
+    const int64_t groups = (p.n_vfull + t - 1) / t + (p.tail ? 1 : 0);
+    return (groups * p.n_tt + cus - 1) / cus * t;
+  };
+  p.tiles = rounds(1) * 103 < rounds(kMaxTiles) * 100 ? 1 : kMaxTiles;
+  p.n_vg = (p.n_vfull + p.tiles - 1) / p.tiles;
   p.partial_bytes = ((size_t)(2 * p.n_vg + 2) * (size_t)N * sizeof(float4) + 255) / 256 * 256;
   p.xt_bytes = ((size_t)N * sizeof(float) + 255) / 256 * 256;
   return p;
@@ -509,25 +552,19 @@ int lm_head_run(const uint16_t* hidden, int64_t N, int64_t K, int64_t hidden_str
   a.n_vfull = p.n_vfull;
   a.n_tt = p.n_tt;
   a.n_vg = p.n_vg;
+  a.tiles = p.tiles;
+  a.tail = p.tail ? 1 : 0;
+  a.blocks = p.blocks;
   a.partial = reinterpret_cast<float4*>(workspace);
   a.logits = out_logits;
   a.ldl = logits_stride;
   float* xt = reinterpret_cast<float*>(reinterpret_cast<unsigned char*>(workspace) + p.partial_bytes);
-  const int64_t grid = (int64_t)p.n_vg * p.n_tt;
+  const int64_t grid = lmh::grid_of(p.n_vg + a.tail, p.n_tt, p.blocks);
   if (grid > 0x7FFFFFFFll) return GTP_ERR_UNSUPPORTED;
-  if (out_logits) {
-    if (grid > 0)
-      launch_timed(lmh::lm_head_lse_kernel<false, true>, dim3((unsigned)grid), dim3(lmh::kThreads), s, a);
-    if (p.tail)
-      hipLaunchKernelGGL((lmh::lm_head_lse_kernel<true, true>), dim3((unsigned)p.n_tt),
-                         dim3(lmh::kThreads), 0, s, a);
-  } else {
-    if (grid > 0)
-      launch_timed(lmh::lm_head_lse_kernel<false, false>, dim3((unsigned)grid), dim3(lmh::kThreads), s, a);
-    if (p.tail)
-      hipLaunchKernelGGL((lmh::lm_head_lse_kernel<true, false>), dim3((unsigned)p.n_tt),
-                         dim3(lmh::kThreads), 0, s, a);
-  }
+  if (out_logits)
+    launch_timed(lmh::lm_head_lse_kernel<true>, dim3((unsigned)grid), dim3(lmh::kThreads), s, a);
+  else
+    launch_timed(lmh::lm_head_lse_kernel<false>, dim3((unsigned)grid), dim3(lmh::kThreads), s, a);
   hipLaunchKernelGGL(lmh::lm_head_target_kernel, dim3((unsigned)((N + 3) / 4)), dim3(256), 0, s,
                      weight, hidden, N, V, K, weight_stride, hidden_stride, targets, targets_int64,
                      xt);
