@@ -2064,6 +2064,7 @@ __global__ __launch_bounds__(kSB) void sampler_hist_kernel(SamplerArgs a) {
 #include "tokpath_sampler_topp.h"
 #include "tokpath_sampler_topp32.h"
 #include "tokpath_sampler_topps.h"
+#include "tokpath_sampler_spread.h"
 
 using namespace gtp;
 
@@ -2210,3 +2211,81 @@ int launch_sampler_general(const SamplerArgs& a, int dtype, int64_t B, hipStream
 }
 
 }  // namespace gtp
+
+namespace {
+// Calls the spread kernels can run: sampling without top-k.
+bool spread_can(int64_t B, int64_t V, const gtp_sampler_params* p) {
+  return B > 0 && B <= 0xFFFF && V > 0 && V <= GTP_SAMPLER_MAX_V && p->temperature > 0.0f &&
+         p->temperature <= 1024.0f && (p->top_k <= 0 || (int64_t)p->top_k >= V);
+}
+}  // namespace
+
+extern "C" size_t gtp_sample_spread_workspace_bytes(int64_t B, int64_t V,
+                                                    const gtp_sampler_params* params) {
+  if (!params || !spread_can(B, V, params)) return 0;
+  return spread::ws_bytes(B, spread::slices(B));
+}
+
+// Where the spread kernels are the faster ones (us, both measured, the other
+// kernel first):
+// - Against the row-wise kernel always: fp16 [2, 151936] 134 / 29, fp16
+//   [256, 248320] 236 / 176, fp32 plain [16, 248320] 258 / 37, [256, 248320]
+//   335 / 218, bf16 [*, 50257] unaligned likewise.
+// - Against the fp32 top-p kernel (two reads by one workgroup per row) up to
+//   96 rows: [8, 151936] 71 / 30, [48, 151936] 80 / 49, [96, 248320] 114 /
+//   103; [160, 151936] 83 / 104.
+// - Against the value-histogram kernel, whose bf16 counts need no weight per
+//   token, up to 16 rows: [2, 151936] plain 45 / 35, [16, 248320] 58 / 55;
+//   [48, 151936] 46 / 62.
+// - Against the bf16 top-p kernels never: [2, 151936] 27 / 29, [16, 151936]
+//   31 / 33, [64, 151936] 34 / 51.
+extern "C" int gtp_sample_spread_wins(int dtype, int64_t B, int64_t V, int aligned,
+                                      int64_t hist_len, int has_mask,
+                                      const gtp_sampler_params* params) {
+  if (!params || dtype < GTP_DTYPE_F32 || dtype > GTP_DTYPE_F16 || hist_len < 0 ||
+      !spread_can(B, V, params))
+    return 0;
+  const GeneralRoute r = route_general(dtype, B, V, aligned != 0, hist_len, has_mask != 0, params,
+                                       true, (size_t)-1);
+  switch (r.route) {
+    case GTP_ROUTE_ROWWISE:
+      return 1;
+    case GTP_ROUTE_TOPP32:
+      return B <= 96;
+    case GTP_ROUTE_HIST:
+      return B <= 16;
+    default:
+      return 0;
+  }
+}
+
+extern "C" int gtp_sample_rows_spread(const void* logits, int dtype, int64_t B, int64_t V,
+                                      int64_t row_stride, const int32_t* history, int64_t hist_len,
+                                      int64_t hist_stride, const uint32_t* allow_mask,
+                                      int64_t mask_stride, const float* uniforms,
+                                      const gtp_sampler_params* params, const uint8_t* finished,
+                                      int64_t pad_token_id, int64_t* out_ids, float* out_logprob,
+                                      float* out_sampled_logprob, int32_t* out_kept,
+                                      float* out_thresh_value, int32_t* out_thresh_id,
+                                      int32_t* out_status, void* workspace, size_t workspace_bytes,
+                                      void* stream) {
+  SamplerArgs a;
+  const int rc = sampler_args(a, logits, dtype, B, V, row_stride, history, hist_len, hist_stride,
+                              allow_mask, mask_stride, uniforms, params, finished, pad_token_id,
+                              out_ids, out_logprob, out_sampled_logprob, out_kept,
+                              out_thresh_value, out_thresh_id, out_status);
+  if (rc != GTP_OK) return rc;
+  if (B == 0) return GTP_OK;
+  if (!spread_can(B, V, params)) return GTP_ERR_UNSUPPORTED;
+  if (!workspace || workspace_bytes < spread::ws_bytes(B, spread::slices(B)))
+    return GTP_ERR_INVALID_ARGUMENT;
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  switch (dtype) {
+    case GTP_DTYPE_BF16:
+      return spread::launch<uint16_t>(a, B, workspace, s);
+    case GTP_DTYPE_F16:
+      return spread::launch<_Float16>(a, B, workspace, s);
+    default:
+      return spread::launch<float>(a, B, workspace, s);
+  }
+}

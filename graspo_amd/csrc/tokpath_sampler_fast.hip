@@ -1521,14 +1521,13 @@ __global__ __launch_bounds__(256) void zero_words_kernel(uint32_t* __restrict__ 
   if (i < n) p[i] = 0u;
 }
 
-int sample_rows_impl(const void* logits, int dtype, int64_t B, int64_t V, int64_t row_stride,
-                     const int32_t* history, int64_t hist_len, int64_t hist_stride,
-                     const uint32_t* allow_mask, int64_t mask_stride, const float* uniforms,
-                     const gtp_sampler_params* params, const uint8_t* finished,
-                     int64_t pad_token_id, int64_t* out_ids, float* out_logprob,
-                     float* out_sampled_logprob, int32_t* out_kept, float* out_thresh_value,
-                     int32_t* out_thresh_id, int32_t* out_status, void* workspace,
-                     size_t workspace_bytes, bool clear_counters, void* stream) {
+int sampler_args(SamplerArgs& a, const void* logits, int dtype, int64_t B, int64_t V,
+                 int64_t row_stride, const int32_t* history, int64_t hist_len, int64_t hist_stride,
+                 const uint32_t* allow_mask, int64_t mask_stride, const float* uniforms,
+                 const gtp_sampler_params* params, const uint8_t* finished, int64_t pad_token_id,
+                 int64_t* out_ids, float* out_logprob, float* out_sampled_logprob,
+                 int32_t* out_kept, float* out_thresh_value, int32_t* out_thresh_id,
+                 int32_t* out_status) {
   if (!params || B < 0 || V <= 0 || row_stride < V) return GTP_ERR_INVALID_ARGUMENT;
   if (dtype != GTP_DTYPE_F32 && dtype != GTP_DTYPE_BF16 && dtype != GTP_DTYPE_F16)
     return GTP_ERR_INVALID_ARGUMENT;
@@ -1539,10 +1538,7 @@ int sample_rows_impl(const void* logits, int dtype, int64_t B, int64_t V, int64_
   if (allow_mask && mask_stride < (V + 31) / 32) return GTP_ERR_INVALID_ARGUMENT;
   if (hist_len < 0) return GTP_ERR_INVALID_ARGUMENT;
   if (history && hist_len > 0 && hist_stride < hist_len) return GTP_ERR_INVALID_ARGUMENT;
-  const bool greedy = !(params->temperature > 0.0f);
-  if (!greedy && B > 0 && !uniforms) return GTP_ERR_INVALID_ARGUMENT;
-  if (B == 0) return GTP_OK;
-  SamplerArgs a;
+  if (params->temperature > 0.0f && B > 0 && !uniforms) return GTP_ERR_INVALID_ARGUMENT;
   a.logits = logits;
   a.V = V;
   a.row_stride = row_stride;
@@ -1565,6 +1561,25 @@ int sample_rows_impl(const void* logits, int dtype, int64_t B, int64_t V, int64_
   a.out_tv = out_thresh_value;
   a.out_tid = out_thresh_id;
   a.out_status = out_status;
+  return GTP_OK;
+}
+
+int sample_rows_impl(const void* logits, int dtype, int64_t B, int64_t V, int64_t row_stride,
+                     const int32_t* history, int64_t hist_len, int64_t hist_stride,
+                     const uint32_t* allow_mask, int64_t mask_stride, const float* uniforms,
+                     const gtp_sampler_params* params, const uint8_t* finished,
+                     int64_t pad_token_id, int64_t* out_ids, float* out_logprob,
+                     float* out_sampled_logprob, int32_t* out_kept, float* out_thresh_value,
+                     int32_t* out_thresh_id, int32_t* out_status, void* workspace,
+                     size_t workspace_bytes, bool clear_counters, void* stream) {
+  SamplerArgs a;
+  const int arc = sampler_args(a, logits, dtype, B, V, row_stride, history, hist_len, hist_stride,
+                               allow_mask, mask_stride, uniforms, params, finished, pad_token_id,
+                               out_ids, out_logprob, out_sampled_logprob, out_kept,
+                               out_thresh_value, out_thresh_id, out_status);
+  if (arc != GTP_OK) return arc;
+  if (B == 0) return GTP_OK;
+  const bool greedy = !(params->temperature > 0.0f);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
 
   const int es = elem_size(dtype);

@@ -32,6 +32,15 @@ struct SamplerArgs {
   int32_t* out_status;
 };
 
+// Checks a sampling call's arguments (every entry point's) and collects them.
+int sampler_args(SamplerArgs& a, const void* logits, int dtype, int64_t B, int64_t V,
+                 int64_t row_stride, const int32_t* history, int64_t hist_len, int64_t hist_stride,
+                 const uint32_t* allow_mask, int64_t mask_stride, const float* uniforms,
+                 const gtp_sampler_params* params, const uint8_t* finished, int64_t pad_token_id,
+                 int64_t* out_ids, float* out_logprob, float* out_sampled_logprob,
+                 int32_t* out_kept, float* out_thresh_value, int32_t* out_thresh_id,
+                 int32_t* out_status);
+
 // One workgroup of 1024 threads per row (any layout, V <= GTP_SAMPLER_MAX_V),
 // or, for small batches of bf16 top-p rows, S workgroups per row that merge
 // their counts through `workspace` (topp_workspace_bytes of it, zeroed once).

@@ -73,6 +73,12 @@ void* sampler_workspace(const at::Tensor& like, size_t bytes, int64_t stream) {
   return ws.data_ptr();
 }
 
+// 16-byte aligned logits and row stride
+bool rows_aligned(const at::Tensor& logits) {
+  return (reinterpret_cast<uintptr_t>(logits.data_ptr()) & 15u) == 0 &&
+         ((uint64_t)(row_stride_of(logits) * logits.element_size()) & 15u) == 0;
+}
+
 using SampleOut =
     std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor, at::Tensor, at::Tensor, at::Tensor>;
 
@@ -143,15 +149,21 @@ SampleOut sample(const at::Tensor& logits, double temperature, int64_t top_k, do
   p.top_k = (int32_t)top_k;
   p.top_p = (float)top_p;
   p.repetition_penalty = (float)repetition_penalty;
-  const size_t ws_bytes = gtp_sample_workspace_bytes(dtype_code(logits), B, V, &p);
-  void* ws = sampler_workspace(logits, ws_bytes, stream);
-  const int rc = gtp_sample_rows(
-      logits.data_ptr(), dtype_code(logits), B, V, row_stride_of(logits), hist, hist_len,
+  const int dt = dtype_code(logits);
+  const bool spread = gtp_sample_spread_wins(dt, B, V, rows_aligned(logits), hist_len,
+                                             mask != nullptr, &p) != 0;
+  at::Tensor own;  // the spread kernels' workspace carries nothing between calls
+  const size_t ws_bytes = spread ? gtp_sample_spread_workspace_bytes(B, V, &p)
+                                 : gtp_sample_workspace_bytes(dt, B, V, &p);
+  if (spread) own = at::empty({(int64_t)ws_bytes}, opt.dtype(at::kByte));
+  void* ws = spread ? own.data_ptr() : sampler_workspace(logits, ws_bytes, stream);
+  const int rc = (spread ? gtp_sample_rows_spread : gtp_sample_rows)(
+      logits.data_ptr(), dt, B, V, row_stride_of(logits), hist, hist_len,
       hist_stride, mask, mask_stride, u, &p, fin, pad_token_id, ids.data_ptr<int64_t>(),
       lp.data_ptr<float>(), slp.data_ptr<float>(), kept.data_ptr<int32_t>(), tv.data_ptr<float>(),
       tid.data_ptr<int32_t>(), st.data_ptr<int32_t>(), ws, ws_bytes,
       reinterpret_cast<void*>(stream));
-  check_rc(rc, "gtp_sample_rows");
+  check_rc(rc, spread ? "gtp_sample_rows_spread" : "gtp_sample_rows");
   return {ids, lp, slp, kept, tv, tid, st};
 }
 
@@ -172,14 +184,25 @@ std::tuple<int64_t, int64_t> sample_route(const at::Tensor& logits, double tempe
   p.repetition_penalty = (float)repetition_penalty;
   const int dt = dtype_code(logits);
   const size_t ws_bytes = gtp_sample_workspace_bytes(dt, B, V, &p);
-  const int64_t es = logits.element_size();
-  const bool aligned = (reinterpret_cast<uintptr_t>(logits.data_ptr()) & 15u) == 0 &&
-                       ((uint64_t)(row_stride_of(logits) * es) & 15u) == 0;
   int32_t route = 0, slices = 0;
-  check_rc(gtp_sample_route(dt, B, V, aligned ? 1 : 0, hist_len, has_mask ? 1 : 0, &p, ws_bytes,
+  check_rc(gtp_sample_route(dt, B, V, rows_aligned(logits) ? 1 : 0, hist_len, has_mask ? 1 : 0, &p, ws_bytes,
                             &route, &slices),
            "gtp_sample_route");
   return {route, slices};
+}
+
+// Whether `sample` runs the spread kernels for these logits and parameters
+// (then not sample_route's).
+bool sample_spread(const at::Tensor& logits, double temperature, int64_t top_k, double top_p,
+                   double repetition_penalty, int64_t hist_len, bool has_mask) {
+  check_rows(logits, "logits");
+  gtp_sampler_params p;
+  p.temperature = (float)temperature;
+  p.top_k = (int32_t)top_k;
+  p.top_p = (float)top_p;
+  p.repetition_penalty = (float)repetition_penalty;
+  return gtp_sample_spread_wins(dtype_code(logits), logits.size(0), logits.size(1),
+                                rows_aligned(logits), hist_len, has_mask, &p) != 0;
 }
 
 const void* targets_ptr(const at::Tensor& logits, const at::Tensor& targets, int64_t N,
@@ -726,6 +749,10 @@ TORCH_LIBRARY(graspo_tokpath, m) {
       "sample_route(Tensor logits, float temperature, int top_k, float top_p, "
       "float repetition_penalty, int hist_len, bool has_mask) -> (int, int)",
       &sample_route);
+  m.def(
+      "sample_spread(Tensor logits, float temperature, int top_k, float top_p, "
+      "float repetition_penalty, int hist_len, bool has_mask) -> bool",
+      &sample_spread);
   m.def("logprob_entropy(Tensor logits, Tensor targets, int stream) -> (Tensor, Tensor, Tensor)",
         &logprob_entropy);
   m.def(

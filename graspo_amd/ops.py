@@ -104,13 +104,23 @@ ROUTE_SPLIT_TOPK, ROUTE_TOPP_SPLIT, ROUTE_TOPP, ROUTE_TOPP32, ROUTE_HIST, ROUTE_
 def sample_route(logits: torch.Tensor, *, temperature: float, top_k: int = 0,
                  top_p: float = 1.0, repetition_penalty: float = 1.0, hist_len: int = 0,
                  has_mask: bool = False) -> tuple[int, int]:
-    """(ROUTE_*, workgroups per row) of the kernel :func:`sample` would run for
-    these logits and parameters (gtp_sample_route, with the workspace the op
-    passes).  Host-only: launches nothing."""
+    """(ROUTE_*, workgroups per row) of the kernel that gtp_sample_rows would
+    run for these logits and parameters (gtp_sample_route, with the workspace
+    the op passes); :func:`sample` takes the spread kernels instead where
+    :func:`sample_spread` says so.  Host-only: launches nothing."""
     ops = load()
     logits = _as_rows(logits)
     return tuple(ops.sample_route(logits, float(temperature), int(top_k), float(top_p),
                                   float(repetition_penalty), int(hist_len), bool(has_mask)))
+
+
+def sample_spread(logits: torch.Tensor, *, temperature: float, top_k: int = 0, top_p: float = 1.0,
+                  repetition_penalty: float = 1.0, hist_len: int = 0,
+                  has_mask: bool = False) -> bool:
+    """Whether :func:`sample` runs the spread kernels (gtp_sample_rows_spread)
+    for these logits and parameters.  Host-only."""
+    return load().sample_spread(_as_rows(logits), float(temperature), int(top_k), float(top_p),
+                                float(repetition_penalty), int(hist_len), bool(has_mask))
 
 
 def logprob_entropy(logits: torch.Tensor, targets: torch.Tensor):

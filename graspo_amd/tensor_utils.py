@@ -17,10 +17,12 @@ from torch.nn import functional as F  # noqa: N812
 from . import ops
 
 
-def _fp32_top_p_kernel_takes(logits: torch.Tensor, temperature: float, top_k: int,
-                             top_p: float) -> bool:
-    """Whether an fp32 call without history or mask goes to the fp32 top-p
-    kernel, as the library's own routing decides (gtp_sample_route)."""
+def _fp32_kernel_takes(logits: torch.Tensor, temperature: float, top_k: int,
+                       top_p: float) -> bool:
+    """Whether an fp32 call without history or mask goes to the spread or the
+    fp32 top-p kernels, as the library's own routing decides."""
+    if ops.sample_spread(logits, temperature=temperature, top_k=top_k, top_p=top_p):
+        return True
     route, _ = ops.sample_route(logits, temperature=temperature, top_k=top_k, top_p=top_p)
     return route == ops.ROUTE_TOPP32
 
@@ -29,15 +31,15 @@ def _bf16_when_exact(logits: torch.Tensor, temperature: float, top_k: int,
                      top_p: float = 1.0) -> torch.Tensor:
     """fp32 rows as their bf16 copy when every value is a bf16 value -- the
     reference's callers pass ``logits.float()`` of a bf16 model -- and the
-    call would otherwise take the row-wise kernel (sampling without a top-k
-    of at most 128, other than the top-p rows the fp32 top-p kernel reads
-    directly, which is faster than the narrowing and its host
-    synchronisation): the value-histogram kernel takes bf16 rows only, and
+    call would otherwise take the row-wise kernel (sampling with a top-k above
+    128; the spread and the fp32 top-p kernels read the rows directly, which
+    is faster than the narrowing and its host synchronisation): the
+    value-histogram kernel takes bf16 rows only, and
     the samples are the same because the float inputs are.  Costs one pass
     over the rows and one host synchronisation."""
     if (logits.dtype != torch.float32 or logits.dim() != 2 or not logits.is_cuda
             or not temperature > 0 or 1 <= top_k <= 128
-            or _fp32_top_p_kernel_takes(logits, temperature, top_k, top_p)):
+            or _fp32_kernel_takes(logits, temperature, top_k, top_p)):
         return logits
     bf, inexact = ops.to_bf16_exact(logits)
     return bf if int(inexact) == 0 else logits

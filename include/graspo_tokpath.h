@@ -180,6 +180,35 @@ int gtp_sample_route(int dtype, int64_t B, int64_t V, int aligned, int64_t hist_
                      int has_mask, const gtp_sampler_params* params, size_t workspace_bytes,
                      int32_t* out_route, int32_t* out_slices);
 
+/*
+ * gtp_sample_rows_spread -- gtp_sample_rows for sampling calls without top-k
+ * (T > 0, top_k <= 0 or >= V), every row spread over several workgroups in
+ * three launches, any dtype, alignment and vocabulary; the same arguments and
+ * bit-exact results.  The workspace is required
+ * (gtp_sample_spread_workspace_bytes, 0 for a call it does not take), 256-byte
+ * aligned, no contents carried between calls.
+ * gtp_sample_spread_wins tells whether it is the faster one for a call
+ * (aligned, hist_len and has_mask as in gtp_sample_route); the torch op asks
+ * it.
+ *
+ * Replaces the reference's per-step sampler on small batches
+ *   _next_token_from_logits  src/graspo/backends/graspoflow/tensor_utils.py:649-658
+ *   _sample_next_token       src/graspo/backends/graspoflow/tensor_utils.py:671-683
+ */
+int gtp_sample_rows_spread(const void* logits, int dtype, int64_t B, int64_t V,
+                           int64_t row_stride, const int32_t* history, int64_t hist_len,
+                           int64_t hist_stride, const uint32_t* allow_mask,
+                           int64_t mask_stride, const float* uniforms,
+                           const gtp_sampler_params* params, const uint8_t* finished,
+                           int64_t pad_token_id, int64_t* out_ids, float* out_logprob,
+                           float* out_sampled_logprob, int32_t* out_kept,
+                           float* out_thresh_value, int32_t* out_thresh_id,
+                           int32_t* out_status, void* workspace, size_t workspace_bytes,
+                           void* stream);
+size_t gtp_sample_spread_workspace_bytes(int64_t B, int64_t V, const gtp_sampler_params* params);
+int gtp_sample_spread_wins(int dtype, int64_t B, int64_t V, int aligned, int64_t hist_len,
+                           int has_mask, const gtp_sampler_params* params);
+
 /* Size of the library's own workspace for gtp_sample_rows_noalloc. */
 #define GTP_NOALLOC_SCRATCH_BYTES ((size_t)8 << 20)
 
