@@ -2065,6 +2065,7 @@ __global__ __launch_bounds__(kSB) void sampler_hist_kernel(SamplerArgs a) {
 #include "tokpath_sampler_topp32.h"
 #include "tokpath_sampler_topps.h"
 #include "tokpath_sampler_spread.h"
+#include "tokpath_sampler_greedy.h"
 
 using namespace gtp;
 

@@ -1392,6 +1392,21 @@ FastPlan plan_fast(int dtype, int64_t B, int64_t V, const gtp_sampler_params* p,
   return pl;
 }
 
+// Greedy rows that the greedy kernel takes, of any alignment.  The row-wise
+// kernel keeps the smallest vocabularies and the largest batches.  With a mask
+// or a penalty the split kernel keeps the aligned rows that fill the chip with
+// one workgroup each: it tests a vector against its threshold where the greedy
+// kernel penalises and masks every token (bf16 [256, 151936], split / greedy:
+// mask 21.7 / 26.6 us, penalty 18.9 / 30.5; [255, 151936], in slices, 53.3 /
+// 29.2 and 49.5 / 33.9; [64, 151936] 21.8 / 17.0 and 20.7 / 19.7).
+bool greedy_takes(int dtype, int64_t B, int64_t V, const gtp_sampler_params* p, bool aligned,
+                  int64_t hist_len, bool has_mask) {
+  if (p->temperature > 0.0f || V < 512 || V > GTP_SAMPLER_MAX_V || B < 1 || B > 0xFFFF) return false;
+  if (!has_mask && (hist_len == 0 || p->repetition_penalty == 1.0f)) return true;
+  const FastPlan pl = plan_fast(dtype, B, V, p, aligned);
+  return !pl.fast || pl.S > 1;
+}
+
 }  // namespace gtp
 
 using namespace gtp;
@@ -1410,6 +1425,12 @@ extern "C" int gtp_sample_route(int dtype, int64_t B, int64_t V, int aligned, in
   if (dtype != GTP_DTYPE_F32 && dtype != GTP_DTYPE_BF16 && dtype != GTP_DTYPE_F16)
     return GTP_ERR_INVALID_ARGUMENT;
   if (V > GTP_SAMPLER_MAX_V || B > 0x7FFFFFFFll) return GTP_ERR_UNSUPPORTED;
+  if (greedy_takes(dtype, B, V, params, aligned != 0, hist_len, has_mask != 0)) {
+    const size_t need = plan_fast(dtype, B, V, params, true).ws_bytes;
+    *out_route = GTP_ROUTE_SPLIT_TOPK;
+    if (out_slices) *out_slices = greedy_slices(B, V, need > 0 && workspace_bytes >= need);
+    return GTP_OK;
+  }
   const FastPlan pl = plan_fast(dtype, B, V, params, aligned != 0);
   if (pl.fast) {
     *out_route = GTP_ROUTE_SPLIT_TOPK;
@@ -1587,7 +1608,9 @@ int sample_rows_impl(const void* logits, int dtype, int64_t B, int64_t V, int64_
   const bool aligned = (reinterpret_cast<uintptr_t>(logits) & 15u) == 0 &&
                        (((uint64_t)row_stride * (uint64_t)es) & 15u) == 0;
   const FastPlan pl = plan_fast(dtype, B, V, params, aligned);
-  if (!pl.fast) {
+  const bool greedy_row =
+      greedy_takes(dtype, B, V, params, aligned, a.hist_len, allow_mask != nullptr);
+  if (!pl.fast && !greedy_row) {
     const size_t tw = topp_workspace_bytes(dtype, B, V, params, workspace_bytes);
     if (clear_counters && tw > 0 && workspace && workspace_bytes >= tw) {
       // the split top-p kernel's zero region (its per-row arrival counters)
@@ -1599,11 +1622,20 @@ int sample_rows_impl(const void* logits, int dtype, int64_t B, int64_t V, int64_
   }
   if (pl.ws_bytes > 0 && (!workspace || workspace_bytes < pl.ws_bytes))
     return GTP_ERR_INVALID_ARGUMENT;
-  if (clear_counters && pl.ws_bytes > 0) {
-    const int64_t nw = (int64_t)(pl.cnt_bytes / 4);
+  // greedy rows split where an aligned call of their size has a workspace
+  // (its slots, 2 KB per slice of at most 8, hold the greedy slices' 32 bytes)
+  const FastPlan gp = greedy_row ? plan_fast(dtype, B, V, params, true) : pl;
+  const bool has_ws = gp.ws_bytes > 0 && workspace && workspace_bytes >= gp.ws_bytes;
+  if (clear_counters && has_ws) {
+    const int64_t nw = (int64_t)(gp.cnt_bytes / 4);
     hipLaunchKernelGGL(zero_words_kernel, dim3((unsigned)((nw + 255) / 256)), dim3(256), 0, st,
                        reinterpret_cast<uint32_t*>(workspace), nw);
   }
+  if (greedy_row)
+    return launch_greedy(a, dtype, B, greedy_slices(B, V, has_ws), workspace,
+                         has_ws ? reinterpret_cast<unsigned char*>(workspace) + gp.cnt_bytes
+                                : nullptr,
+                         st);
 
   FastArgs fa;
   fa.a = a;

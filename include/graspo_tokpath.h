@@ -170,7 +170,7 @@ size_t gtp_sample_workspace_bytes(int dtype, int64_t B, int64_t V,
  *   workspace_bytes  the workspace the call would pass (0: none)
  * out_route gets one of GTP_ROUTE_*, out_slices the workgroups per row.
  */
-#define GTP_ROUTE_SPLIT_TOPK 1  /* greedy / top-k <= 128: split sampler      */
+#define GTP_ROUTE_SPLIT_TOPK 1  /* greedy, top-k <= 128: one read, split     */
 #define GTP_ROUTE_TOPP_SPLIT 2  /* bf16 top-p rows of small batches, split   */
 #define GTP_ROUTE_TOPP 3        /* bf16 top-p rows, one workgroup per row    */
 #define GTP_ROUTE_TOPP32 4      /* fp32 top-p rows, one workgroup per row    */

@@ -1,0 +1,98 @@
+"""The greedy kernel against the oracle, bit for bit: slice counts (one
+workgroup per row and split rows), vocabularies around the slices' edges,
+unaligned rows, masks, penalties, ties across slices, and rows of non-finite
+or no allowed values."""
+
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from tests import _capi
+from tests._util import oracle_sample
+
+DEV = torch.device("cuda:0")
+INTS = ("ids", "kept", "thresh_id", "status")
+
+
+def _mask(B, V, g, density):
+    W = (V + 31) // 32
+    bits = torch.rand(B, W * 32, generator=g) < density
+    bits[:, V:] = False
+    w = (bits.view(B, W, 32).long() << torch.arange(32)).sum(-1)
+    return torch.where(w >= 2**31, w - 2**32, w).to(torch.int32)
+
+
+def _check(x, workspace=True, **kw):
+    L = _capi.lib()
+    ref = oracle_sample(x, temperature=0.0, **kw)
+    gk = {k: (v.to(DEV) if isinstance(v, torch.Tensor) else v) for k, v in kw.items()}
+    st = x.stride(0)
+    buf = torch.empty(x.storage_offset() + x.shape[0] * st + 8, dtype=x.dtype, device=DEV)
+    xd = buf.as_strided(x.shape, (st, 1), x.storage_offset())
+    xd.copy_(x)
+    args, p, B = _capi.sample_args(xd, temperature=0.0, **gk)
+    n = L.gtp_sample_workspace_bytes(_capi.DTYPE[x.dtype], B, x.shape[1], ctypes.byref(p))
+    ws = torch.zeros(max(n, 256) if workspace else 0, dtype=torch.uint8, device=DEV)
+    for _ in range(2):  # the second call finds the counters that the first one left
+        out = _capi.SampleBuffers(B, DEV)
+        assert L.gtp_sample_rows(*args, *out.out_args(), ws.data_ptr() if workspace else None,
+                                 ws.numel(), _capi.stream_handle()) == 0
+        torch.cuda.synchronize()
+        got = out.cpu()
+        for f in INTS:
+            assert np.array_equal(got[f].numpy(), getattr(ref, f)), f
+        assert np.array_equal(got["thresh_value"].numpy().view(np.int32)[ref.status == 0],
+                              ref.thresh_value.view(np.int32)[ref.status == 0])
+        # fp32 sums: 1e-5 of a logprob of at most about 30
+        a, b = got["logprob"].numpy(), ref.logprob
+        assert np.array_equal(np.isnan(a), np.isnan(b))
+        fin = np.isfinite(b)
+        assert np.abs(a[fin] - b[fin]).max(initial=0) <= 1e-3
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,V", [(1, 512), (3, 4103), (1, 151936), (70, 32775), (2, 262144),
+                                 (257, 2055)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("extra", ["plain", "pen", "mask", "pen_mask"])
+def test_greedy_matches_oracle(B, V, dtype, extra):
+    print(B, V, dtype, extra, flush=True)
+    g = torch.Generator().manual_seed(B * 1000 + V)
+    # coarse values: exact ties of the maximum within and across slices
+    x = (torch.randn(B, V + 1, generator=g) * 4).round().div(2).to(dtype)
+    x = x[:, 1:] if V % 2 else x[:, :V]  # rows at odd elements
+    kw = {}
+    if "pen" in extra:
+        kw.update(repetition_penalty=1.3 if V % 3 else 0.7,
+                  history=torch.randint(-1, V, (B, 300), generator=g, dtype=torch.int32))
+    if "mask" in extra:
+        kw["allow_mask"] = _mask(B, V, g, 0.02)
+    _check(x, **kw)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("workspace", [True, False])
+@pytest.mark.parametrize("V", [513, 40003])
+def test_greedy_special_rows(workspace, V):
+    g = torch.Generator().manual_seed(V)
+    x = torch.randn(10, V, generator=g)
+    x[0, V - 1] = float("nan")
+    x[1, 7] = float("inf")
+    x[2] = float("-inf")
+    x[3, :] = float("-inf")
+    x[3, V - 2] = -3.0
+    x[4] = 0.0
+    x[4, ::3] = -0.0  # the two zeros tie
+    x[5, 400] = float("nan")
+    x[6, 11] = 3e38   # overflows under the penalty
+    h = torch.full((10, 4), -1, dtype=torch.int32)
+    h[6, 0] = 11
+    h[7, 3] = V       # a history id beyond the vocabulary
+    for rho in (1.0, 0.5):
+        _check(x, workspace=workspace, history=h, repetition_penalty=rho)
+    m = torch.full((10, (V + 31) // 32), -1, dtype=torch.int32)
+    m[8] = 0          # nothing allowed
+    m[5, 400 // 32] = 0  # the NaN is not allowed
+    _check(x, workspace=workspace, history=h, repetition_penalty=0.5, allow_mask=m)
