@@ -1398,7 +1398,7 @@ FastPlan plan_fast(int dtype, int64_t B, int64_t V, const gtp_sampler_params* p,
 // one workgroup each: it tests a vector against its threshold where the greedy
 // kernel penalises and masks every token (bf16 [256, 151936], split / greedy:
 // mask 21.7 / 26.6 us, penalty 18.9 / 30.5; [255, 151936], in slices, 53.3 /
-// 29.2 and 49.5 / 33.9; [64, 151936] 21.8 / 17.0 and 20.7 / 19.7).
+// 32.2 and 49.5 / 36.0; [64, 151936] 21.8 / 11.4 and 20.7 / 13.0).
 bool greedy_takes(int dtype, int64_t B, int64_t V, const gtp_sampler_params* p, bool aligned,
                   int64_t hist_len, bool has_mask) {
   if (p->temperature > 0.0f || V < 512 || V > GTP_SAMPLER_MAX_V || B < 1 || B > 0xFFFF) return false;
@@ -1426,9 +1426,9 @@ extern "C" int gtp_sample_route(int dtype, int64_t B, int64_t V, int aligned, in
     return GTP_ERR_INVALID_ARGUMENT;
   if (V > GTP_SAMPLER_MAX_V || B > 0x7FFFFFFFll) return GTP_ERR_UNSUPPORTED;
   if (greedy_takes(dtype, B, V, params, aligned != 0, hist_len, has_mask != 0)) {
-    const size_t need = plan_fast(dtype, B, V, params, true).ws_bytes;
+    const FastPlan gp = plan_fast(dtype, B, V, params, true);
     *out_route = GTP_ROUTE_SPLIT_TOPK;
-    if (out_slices) *out_slices = greedy_slices(B, V, need > 0 && workspace_bytes >= need);
+    if (out_slices) *out_slices = gp.ws_bytes > 0 && workspace_bytes >= gp.ws_bytes ? gp.S : 1;
     return GTP_OK;
   }
   const FastPlan pl = plan_fast(dtype, B, V, params, aligned != 0);
@@ -1623,7 +1623,7 @@ int sample_rows_impl(const void* logits, int dtype, int64_t B, int64_t V, int64_
   if (pl.ws_bytes > 0 && (!workspace || workspace_bytes < pl.ws_bytes))
     return GTP_ERR_INVALID_ARGUMENT;
   // greedy rows split where an aligned call of their size has a workspace
-  // (its slots, 2 KB per slice of at most 8, hold the greedy slices' 32 bytes)
+  // (its slots, 2 KB per slice, hold the greedy slices' 32 bytes)
   const FastPlan gp = greedy_row ? plan_fast(dtype, B, V, params, true) : pl;
   const bool has_ws = gp.ws_bytes > 0 && workspace && workspace_bytes >= gp.ws_bytes;
   if (clear_counters && has_ws) {
@@ -1632,7 +1632,8 @@ int sample_rows_impl(const void* logits, int dtype, int64_t B, int64_t V, int64_
                        reinterpret_cast<uint32_t*>(workspace), nw);
   }
   if (greedy_row)
-    return launch_greedy(a, dtype, B, greedy_slices(B, V, has_ws), workspace,
+    return launch_greedy(a, dtype, B, has_ws ? gp.S : 1,
+                         has_ws ? gp.vps * (16 / es) / 8 : (V / 8 + 3) / 4 * 4, workspace,
                          has_ws ? reinterpret_cast<unsigned char*>(workspace) + gp.cnt_bytes
                                 : nullptr,
                          st);

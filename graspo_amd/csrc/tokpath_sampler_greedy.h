@@ -7,12 +7,15 @@
 // a threshold, a pool, a ranking), whose serial steps were most of a small
 // call.  Each row is cut into S slices; every thread folds its tokens into
 // (m, s) and its best (y, id), and the last of the row's workgroups to arrive
-// merges the slices.  Rows may start at any element.
+// merges the slices.  Rows may start at any element.  The slices and their
+// threads' shares are the split kernel's, so a slice of up to four vectors per
+// thread gives the same log-sum-exp to the bit: the logprob of a row that is
+// nearly one-hot, ln(1 + a little), magnifies a unit of the sum.
 //
 // Bound by the latency of a launch, one trip to memory and the arrival on
 // small batches, by the stream on large ones.  bf16 [1, 151936], the split
-// kernel before: 15.5 -> 5.6 us; [64, 151936] 20.6 -> 9.4; [256, 151936] 18.5
-// -> 16.6; fp32 [256, 248320] 71.9 -> 42.7; unaligned bf16 [16, 50257] (the
+// kernel before: 15.5 -> 7.0 us; [64, 151936] 20.6 -> 9.2; [256, 151936] 18.5
+// -> 16.7; fp32 [256, 248320] 71.9 -> 42.7; unaligned bf16 [16, 50257] (the
 // row-wise kernel before) 30.4 -> 7.8.
 #pragma once
 
@@ -21,10 +24,9 @@ namespace greedy {
 
 using spread::put;
 using spread::Range;
-using spread::range_of;
 using spread::take;
 
-constexpr int kMaxS = 16;  // slices per row, one lane each in the merge
+constexpr int kT = 1024;   // threads of a workgroup
 
 // One slice's results (the arrival counters lie elsewhere).
 struct Part {
@@ -57,25 +59,27 @@ __device__ __forceinline__ void finish(const SamplerArgs& a, int64_t b, uint32_t
 }
 
 // kExtra: an allow mask or a penalty.
-template <typename T, int NT, bool kExtra>
-__global__ __launch_bounds__(NT) void sampler_greedy_kernel(SamplerArgs a, uint32_t* ctr,
-                                                            Part* parts) {
+// per: groups of 8 tokens per slice, a multiple of 4.
+template <typename T, bool kExtra>
+__global__ __launch_bounds__(kT) void sampler_greedy_kernel(SamplerArgs a, uint32_t per,
+                                                            uint32_t* ctr, Part* parts) {
   __shared__ uint32_t pen_bits[GTP_SAMPLER_MAX_V / 32];
-  __shared__ unsigned long long red_k[NT / kWave];
-  __shared__ float red[NT / kWave][2];
+  __shared__ unsigned long long red_k[kT / kWave];
+  __shared__ float red[kT / kWave][2];
   const int k = blockIdx.x, S = gridDim.x;
   const int64_t b = blockIdx.y;
   const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
   const T* row = reinterpret_cast<const T*>(a.logits) + b * a.row_stride;
   const uint32_t* mrow = a.mask ? a.mask + b * a.mask_stride : nullptr;
-  const Range r = range_of(a.V, k, S);
+  const uint32_t ng = (uint32_t)(a.V / 8), g0 = min((uint32_t)k * per, ng);
+  const Range r{g0, min(g0 + per, ng), k == S - 1};
   const bool use_pen = kExtra && a.hist_len > 0 && a.rho != 1.0f;
   bool bad = false;
-  if (a.hist_len > 0 && (use_pen || k == 0)) bad = spread::slice_pen(a, b, r, use_pen, pen_bits, NT);
+  if (a.hist_len > 0 && (use_pen || k == 0)) bad = spread::slice_pen(a, b, r, use_pen, pen_bits, kT);
   Lse3 st{kNegInf, 0.0f, 0.0f};
   float by = kNegInf;
   uint32_t bid = 0u;
-  spread::for_groups<T, NT, kExtra>(
+  spread::for_groups<T, kT, kExtra>(
       row, mrow, use_pen ? reinterpret_cast<const uint8_t*>(pen_bits) : nullptr, a.V, r,
       [&](const float(&x)[8], uint32_t id, uint32_t al, uint32_t pb, int n) {
         float y[8];
@@ -118,7 +122,7 @@ __global__ __launch_bounds__(NT) void sampler_greedy_kernel(SamplerArgs a, uint3
   }
   __syncthreads();
   if (wid != 0) return;
-  const bool in = lane < NT / kWave;
+  const bool in = lane < kT / kWave;
   key = wave_max_u64(in ? red_k[lane] : 0ull);
   m = in ? red[lane][0] : kNegInf;
   s = in ? red[lane][1] : 0.0f;
@@ -155,53 +159,34 @@ __global__ __launch_bounds__(NT) void sampler_greedy_kernel(SamplerArgs a, uint3
   finish<T>(a, b, pen_bits, key, m, s, bad);
 }
 
-// Slices per row: one workgroup of 512 threads per CU (two from a quarter
-// of a row per CU on), at least 8 tokens per
-// thread in each; one workgroup of 1024 threads where the chip is full with
-// one row per CU, or without a workspace (`can_split`).  Every workgroup more
-// is one more arrival: bf16 [32, 151936] 8.3 us in 8 slices, 10.2 in 16, 15.1
-// in 32; [64, 151936] 9.4 in 4, 12.2 in 16; [128, 151936] 12.6 in 4, 18.5 in
-// 16; [8, 151936] 6.9 in 16, 8.1 in 32.
-inline int slices(int64_t B, int64_t V, bool can_split) {
-  if (!can_split) return 1;
-  const int64_t cus = device_cus();
-  const int64_t want = ((4 * B > cus ? 2 : 1) * cus + B - 1) / B;
-  const int64_t most = V / (8 * 512);
-  const int64_t S = want < most ? want : most;
-  return (int)(S < 1 ? 1 : S > kMaxS ? kMaxS : S);
-}
-
 template <typename T, bool kExtra>
-void launch_as(const SamplerArgs& a, int64_t B, int S, uint32_t* ctr, Part* parts, hipStream_t s) {
-  const dim3 grid((unsigned)S, (unsigned)B);
-  if (S > 1)
-    launch_timed(sampler_greedy_kernel<T, 512, kExtra>, grid, dim3(512), s, a, ctr, parts);
-  else
-    launch_timed(sampler_greedy_kernel<T, 1024, kExtra>, grid, dim3(1024), s, a, ctr, parts);
+void launch_as(const SamplerArgs& a, int64_t B, int S, uint32_t per, uint32_t* ctr, Part* parts,
+               hipStream_t s) {
+  launch_timed(sampler_greedy_kernel<T, kExtra>, dim3((unsigned)S, (unsigned)B), dim3(kT), s, a, per,
+               ctr, parts);
 }
 
 template <typename T>
-void launch(const SamplerArgs& a, int64_t B, int S, uint32_t* ctr, Part* parts, hipStream_t s) {
+void launch(const SamplerArgs& a, int64_t B, int S, uint32_t per, uint32_t* ctr, Part* parts,
+            hipStream_t s) {
   if (a.mask || (a.hist_len > 0 && a.rho != 1.0f))
-    launch_as<T, true>(a, B, S, ctr, parts, s);
+    launch_as<T, true>(a, B, S, per, ctr, parts, s);
   else
-    launch_as<T, false>(a, B, S, ctr, parts, s);
+    launch_as<T, false>(a, B, S, per, ctr, parts, s);
 }
 
 }  // namespace greedy
 
-int greedy_slices(int64_t B, int64_t V, bool can_split) { return greedy::slices(B, V, can_split); }
-
-int launch_greedy(const SamplerArgs& a, int dtype, int64_t B, int S, void* counters, void* parts,
-                  hipStream_t s) {
+int launch_greedy(const SamplerArgs& a, int dtype, int64_t B, int S, int64_t per, void* counters,
+                  void* parts, hipStream_t s) {
   uint32_t* ctr = reinterpret_cast<uint32_t*>(counters);
   greedy::Part* p = reinterpret_cast<greedy::Part*>(parts);
   if (dtype == GTP_DTYPE_BF16)
-    greedy::launch<uint16_t>(a, B, S, ctr, p, s);
+    greedy::launch<uint16_t>(a, B, S, (uint32_t)per, ctr, p, s);
   else if (dtype == GTP_DTYPE_F16)
-    greedy::launch<_Float16>(a, B, S, ctr, p, s);
+    greedy::launch<_Float16>(a, B, S, (uint32_t)per, ctr, p, s);
   else
-    greedy::launch<float>(a, B, S, ctr, p, s);
+    greedy::launch<float>(a, B, S, (uint32_t)per, ctr, p, s);
   return hipGetLastError() == hipSuccess ? GTP_OK : GTP_ERR_LAUNCH;
 }
 

@@ -85,13 +85,11 @@ GeneralRoute route_general(int dtype, int64_t B, int64_t V, bool aligned, int64_
                            bool has_mask, const gtp_sampler_params* p, bool has_ws,
                            size_t workspace_bytes);
 
-// The greedy kernel (tokpath_sampler_greedy.h): workgroups per row, more than
-// one only where the call brings a workspace (can_split), and its launch.
-// counters: B zero words that the kernel leaves at zero; parts: 32 bytes per
-// slice.
-int greedy_slices(int64_t B, int64_t V, bool can_split);
-int launch_greedy(const SamplerArgs& a, int dtype, int64_t B, int S, void* counters, void* parts,
-                  hipStream_t s);
+// The greedy kernel (tokpath_sampler_greedy.h): S slices of `per` groups of 8
+// tokens (a multiple of 4) per row.  S > 1: counters are B zero words that the
+// kernel leaves at zero, parts 32 bytes per slice.
+int launch_greedy(const SamplerArgs& a, int dtype, int64_t B, int S, int64_t per, void* counters,
+                  void* parts, hipStream_t s);
 
 // Workspace of the top-p path for these parameters within `cap` bytes: the
 // split top-p kernel's counters, headers and slots (0 when the call takes
