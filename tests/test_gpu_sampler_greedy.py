@@ -96,3 +96,29 @@ def test_greedy_special_rows(workspace, V):
     m[8] = 0          # nothing allowed
     m[5, 400 // 32] = 0  # the NaN is not allowed
     _check(x, workspace=workspace, history=h, repetition_penalty=0.5, allow_mask=m)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B", [0, 1, 3, 5])
+@pytest.mark.parametrize("inference", [False, True])
+def test_outputs_are_tensors_of_their_own(B, inference):
+    """The seven outputs share an allocation, not memory: each is contiguous,
+    keeps its dtype, and writing one in place leaves the others."""
+    from graspo_amd import ops
+
+    x = torch.randn(B, 4096, device=DEV)
+    with torch.inference_mode(inference):
+        out = ops.sample(x, temperature=0.0)
+        assert [t.dtype for t in out] == [torch.int64, torch.float32, torch.float32, torch.int32,
+                                          torch.float32, torch.int32, torch.int32]
+        before = [t.clone() for t in out]
+        assert torch.equal(out.ids, x.argmax(1)) and torch.equal(out.thresh_id, out.ids.int())
+        for i, t in enumerate(out):
+            assert t.shape == (B,) and t.is_contiguous() and t.is_inference() == inference
+            v = t._version if not inference else 0
+            t.fill_(77)
+            assert inference or t._version == v + 1
+            for j, o in enumerate(out):
+                if j > i:
+                    assert torch.equal(o, before[j])
+    assert not any(t.requires_grad for t in out)
