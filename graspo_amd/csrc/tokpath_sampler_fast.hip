@@ -1381,9 +1381,12 @@ FastPlan plan_fast(int dtype, int64_t B, int64_t V, const gtp_sampler_params* p,
   pl.S = (int)S;
   pl.vps = vps;
   if (S > 1) {
-    // the arrival counters of every split call on this device (S > 1 needs
-    // B < CUs) lie in one fixed region before the slots: calls whose B
-    // differs never find another call's slot data in their counters
+    // the arrival counters lie before the slots, in one fixed region for up
+    // to 4096 rows: calls whose B differs never find another call's slot data
+    // in their counters.  A row that needs several slices whatever B is (fp32
+    // above 131072 tokens) splits beyond that too: then the counters reach
+    // into other calls' slots, and the call clears them itself
+    // (sample_rows_impl).
     const int64_t nc = B > cus ? B : cus;
     pl.cnt_bytes = (((size_t)nc * 4 + 255) / 256) * 256;
     if (pl.cnt_bytes < kWsZeroBytes) pl.cnt_bytes = kWsZeroBytes;
@@ -1626,7 +1629,9 @@ int sample_rows_impl(const void* logits, int dtype, int64_t B, int64_t V, int64_
   // (its slots, 2 KB per slice, hold the greedy slices' 32 bytes)
   const FastPlan gp = greedy_row ? plan_fast(dtype, B, V, params, true) : pl;
   const bool has_ws = gp.ws_bytes > 0 && workspace && workspace_bytes >= gp.ws_bytes;
-  if (clear_counters && has_ws) {
+  // counters past the fixed region may hold an earlier call's slot data: read
+  // as arrivals, they would lose a row or merge it before its slices are there
+  if (has_ws && (clear_counters || gp.cnt_bytes > kWsZeroBytes)) {
     const int64_t nw = (int64_t)(gp.cnt_bytes / 4);
     hipLaunchKernelGGL(zero_words_kernel, dim3((unsigned)((nw + 255) / 256)), dim3(256), 0, st,
                        reinterpret_cast<uint32_t*>(workspace), nw);

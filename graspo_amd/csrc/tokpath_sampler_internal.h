@@ -49,10 +49,11 @@ int launch_sampler_general(const SamplerArgs& a, int dtype, int64_t B, hipStream
 
 
 // The first kWsZeroBytes of a sampler workspace are words that every call
-// leaves zero: the split kernel's per-row arrival counters (words 0..B-1,
-// B < CUs) and the split top-p kernel's (word kToppSplitCtrWord + b).
+// leaves zero: the split and greedy kernels' per-row arrival counters (words
+// 0..B-1) and the split top-p kernel's (word kToppSplitCtrWord + b).
 // The kernels' slot data lies after it, so a call never finds another call's
-// slot data in its counters.
+// slot data in its counters; a call of more than kWsZeroBytes / 4 rows, whose
+// counters reach past it, clears them first.
 constexpr size_t kWsZeroBytes = 16384;
 constexpr uint32_t kToppSplitCtrWord = 2048;
 // rows a split top-p call may have (at 128 rows of 248320 the one-workgroup
