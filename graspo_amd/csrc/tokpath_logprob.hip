@@ -147,6 +147,7 @@ struct TokenRows {
   const void* targets;
   int64_t V, S, bstride, rstride, tbstride, trstride, ignore;
   int B, t64, has_ignore;
+  __device__ __forceinline__ int64_t rows() const { return (int64_t)B * S; }
   // (sequence, position) of row n; one sequence needs no division
   __device__ __forceinline__ void at(int64_t n, int64_t& b, int64_t& s) const {
     b = B > 1 ? (uint32_t)n / (uint32_t)S : 0;
@@ -160,6 +161,16 @@ struct TokenRows {
     return load_target(targets, t64, b * tbstride + s * trstride);
   }
 };
+
+// Workgroup of a grid that goes on in y: a launch holds fewer than 2^32 work
+// items in one dimension, 2^24 workgroups of 256.
+constexpr int64_t kGridX = 1 << 23;
+__device__ __forceinline__ int64_t flat_workgroup() {
+  return blockIdx.x + (int64_t)blockIdx.y * gridDim.x;
+}
+inline dim3 flat_grid(int64_t n) {
+  return n <= kGridX ? dim3((unsigned)n) : dim3((unsigned)kGridX, (unsigned)((n + kGridX - 1) / kGridX));
+}
 
 // What a row's state gives: logprob, entropy and status.
 struct TokenOut {
@@ -219,8 +230,10 @@ __global__ __launch_bounds__(kLpBlock) void token_logprob_kernel(TokenRows a, To
                                                                  uint32_t* __restrict__ ctr,
                                                                  float* __restrict__ partial) {
   __shared__ float red[kLpBlock / kWave][3];
-  const int64_t n = slices > 1 ? blockIdx.x / (uint32_t)slices : blockIdx.x;
-  const int k = (int)(blockIdx.x - n * slices);
+  // (rows in slices are few: one dimension)
+  const int64_t n = slices > 1 ? blockIdx.x / (uint32_t)slices : flat_workgroup();
+  if (n >= a.rows()) return;
+  const int k = slices > 1 ? (int)(blockIdx.x - n * slices) : 0;
   int64_t b, s;
   a.at(n, b, s);
   const T* row = a.row<T>(b, s);
@@ -448,7 +461,8 @@ __global__ __launch_bounds__(kLpBlock) void token_logprob_backward_kernel(
     TokenRows a, int64_t St, const float* __restrict__ lp, const float* __restrict__ grad_lp,
     const int64_t* __restrict__ count, T* __restrict__ grad, int64_t gbstride, int64_t grstride,
     int slices) {
-  const int64_t n = slices > 1 ? blockIdx.x / (uint32_t)slices : blockIdx.x;
+  const int64_t n = slices > 1 ? blockIdx.x / (uint32_t)slices : flat_workgroup();
+  if (n >= a.rows()) return;
   int64_t b, s;
   a.at(n, b, s);
   const T* row = a.row<T>(b, s);
@@ -464,7 +478,7 @@ __global__ __launch_bounds__(kLpBlock) void token_logprob_backward_kernel(
     }
   }
   logprob_backward_slice<T>(row, a.V, tgt, g, lse, grad + b * gbstride + s * grstride,
-                            (int)(blockIdx.x - n * slices), slices);
+                            slices > 1 ? (int)(blockIdx.x - n * slices) : 0, slices);
 }
 
 // loss = -sum_n lp_n v_n / count, count = sum_n v_n, v_n = 1 unless row n is
@@ -599,7 +613,7 @@ void targets_launch(const TokenRows& a, int64_t N, uint32_t* ctr, int n_ctr, con
 template <typename T>
 void token_logprob_launch(const TokenRows& a, const TokenOut& out, int64_t N, int slices,
                           uint32_t* ctr, hipStream_t s) {
-  const dim3 grid((unsigned)(N * slices)), block(kLpBlock);
+  const dim3 grid = flat_grid(N * slices), block(kLpBlock);
   float* partial = reinterpret_cast<float*>(ctr + (slices > 1 ? N : 0));
   if (out.H)
     launch_timed(token_logprob_kernel<T, true>, grid, block, s, a, out, slices, ctr, partial);
@@ -614,7 +628,7 @@ int token_rows(const gtp_token_rows* r, TokenRows& a, bool need_targets = true) 
       r->batch_stride < 0 || r->row_stride < 0 || r->target_batch_stride < 0 ||
       r->target_row_stride < 0 || r->dtype < GTP_DTYPE_F32 || r->dtype > GTP_DTYPE_F16)
     return GTP_ERR_INVALID_ARGUMENT;
-  if (r->B > 0x3FFFFFFll || r->S > 0x3FFFFFFll || (r->B > 0 && r->S > 0x3FFFFFFll / r->B) ||
+  if (r->B > 0x7FFFFFFFll || r->S > 0x7FFFFFFFll || (r->B > 0 && r->S > 0x7FFFFFFFll / r->B) ||
       r->V > 0x7FFFFFFFll)
     return GTP_ERR_UNSUPPORTED;
   if (r->B > 0 && r->S > 0 && (!r->logits || (need_targets && !r->targets)))
@@ -755,7 +769,7 @@ extern "C" int gtp_token_logprob_backward(const gtp_token_rows* rows, int64_t po
   if (a.B == 1) positions = positions == rows->S ? a.S : positions;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const int slices = row_slices(rows->dtype, N, a.V);
-  const dim3 grid((unsigned)(N * slices)), block(kLpBlock);
+  const dim3 grid = flat_grid(N * slices), block(kLpBlock);
   switch (rows->dtype) {
     case GTP_DTYPE_BF16:
       launch_timed(token_logprob_backward_kernel<uint16_t>, grid, block, s, a, positions, logprob,

@@ -280,6 +280,28 @@ gtp_token_rows token_rows(const at::Tensor& logits, const at::Tensor& targets,
   return r;
 }
 
+uint32_t* verdict_ptr(const at::Tensor& words) {
+  return reinterpret_cast<uint32_t*>(words.data_ptr<int32_t>());
+}
+
+// Pinned words for a look at the targets, each of them pending.
+at::Tensor verdict_words() {
+  at::Tensor words = at::empty({GTP_VERDICT_WORDS},
+                               at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+  for (int i = 0; i < GTP_VERDICT_WORDS; ++i) verdict_ptr(words)[i] = GTP_VERDICT_PENDING;
+  return words;
+}
+
+// Waits for the words of a look that has been launched (or whose launch
+// failed), before anything is raised: given back to the allocator while the
+// kernel may still write them, they would answer for a later call.  Words
+// whose wait fails are kept for good.
+int verdict_wait(const at::Tensor& words, int* found, void* stream) {
+  const int rc = gtp_verdict_wait(verdict_ptr(words), found, stream);
+  if (rc != GTP_OK) new at::Tensor(words);
+  return rc;
+}
+
 // (logprob, entropy or an empty tensor, mean loss, counted rows, whether a
 // target lies outside [0, V)).  mean: also -sum(logprob) / count.  Waits for
 // the look at the targets, which runs ahead of the rows, not for the rows.
@@ -299,24 +321,24 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor, bool> token_logprob(
     loss = at::empty({}, f32);
     count = at::empty({}, f32.dtype(at::kLong));
   }
-  at::Tensor words = at::empty({GTP_VERDICT_WORDS},
-                               at::TensorOptions().dtype(at::kInt).pinned_memory(true));
-  uint32_t* verdict = reinterpret_cast<uint32_t*>(words.data_ptr<int32_t>());
-  for (int i = 0; i < GTP_VERDICT_WORDS; ++i) verdict[i] = GTP_VERDICT_PENDING;
+  const at::Tensor words = verdict_words();
   const size_t ws_bytes = gtp_token_logprob_workspace_bytes(r.dtype, N, r.V);
   at::Tensor ws;
   if (ws_bytes) ws = at::empty({(int64_t)ws_bytes}, logits.options().dtype(at::kByte));
-  check_rc(gtp_token_logprob_rows(&r, lp.data_ptr<float>(), entropy ? H.data_ptr<float>() : nullptr,
-                                  nullptr, verdict, ws_bytes ? ws.data_ptr() : nullptr, ws_bytes,
-                                  st),
-           "gtp_token_logprob_rows");
+  const int rc = gtp_token_logprob_rows(&r, lp.data_ptr<float>(),
+                                        entropy ? H.data_ptr<float>() : nullptr, nullptr,
+                                        verdict_ptr(words), ws_bytes ? ws.data_ptr() : nullptr,
+                                        ws_bytes, st);
+  // an argument error comes before any launch, a launch error after the look's
+  if (rc != GTP_OK && rc != GTP_ERR_LAUNCH) check_rc(rc, "gtp_token_logprob_rows");
   const int mean_rc = mean ? gtp_token_mean_loss(&r, lp.data_ptr<float>(), loss.data_ptr<float>(),
                                                  count.data_ptr<int64_t>(), st)
                            : GTP_OK;
-  // before any other error is raised: the words must outlive the kernel
   int bad = 0;
-  check_rc(gtp_verdict_wait(verdict, &bad, st), "gtp_verdict_wait");
+  const int wait_rc = verdict_wait(words, &bad, st);
+  check_rc(rc, "gtp_token_logprob_rows");
   check_rc(mean_rc, "gtp_token_mean_loss");
+  check_rc(wait_rc, "gtp_verdict_wait");
   return {lp, H, loss, count, bad != 0};
 }
 
@@ -341,14 +363,13 @@ at::Tensor verdict_begin(const at::Tensor& targets, int64_t V, const c10::option
     }
     ++k;
   }
-  at::Tensor words = at::empty({GTP_VERDICT_WORDS},
-                               at::TensorOptions().dtype(at::kInt).pinned_memory(true));
-  uint32_t* verdict = reinterpret_cast<uint32_t*>(words.data_ptr<int32_t>());
-  for (int i = 0; i < GTP_VERDICT_WORDS; ++i) verdict[i] = GTP_VERDICT_PENDING;
-  check_rc(gtp_targets_verdict(targets.data_ptr(), targets.scalar_type() == at::kLong,
-                               targets.size(0), targets.stride(0), V, flags[0], flags[1], verdict,
-                               st),
-           "gtp_targets_verdict");
+  const at::Tensor words = verdict_words();
+  const int rc = gtp_targets_verdict(targets.data_ptr(), targets.scalar_type() == at::kLong,
+                                     targets.size(0), targets.stride(0), V, flags[0], flags[1],
+                                     verdict_ptr(words), st);
+  int found = 0;
+  if (rc == GTP_ERR_LAUNCH) verdict_wait(words, &found, st);
+  check_rc(rc, "gtp_targets_verdict");
   return words;
 }
 
@@ -358,9 +379,7 @@ int64_t verdict_end(const at::Tensor& words, int64_t stream) {
                   words.numel() == GTP_VERDICT_WORDS && words.is_contiguous(),
               "graspo_tokpath.verdict_end: expected verdict_begin's words");
   int found = 0;
-  check_rc(gtp_verdict_wait(reinterpret_cast<const uint32_t*>(words.data_ptr<int32_t>()), &found,
-                            reinterpret_cast<void*>(stream)),
-           "gtp_verdict_wait");
+  check_rc(verdict_wait(words, &found, reinterpret_cast<void*>(stream)), "gtp_verdict_wait");
   return found;
 }
 

@@ -291,7 +291,8 @@ typedef struct gtp_token_rows {
  * GTP_VERDICT_BAD when one of its targets lies outside [0, V).
  * gtp_verdict_wait waits for the words alone (the rows may still be
  * streaming); *found gets 1 for a bad target and 2 for a flag, or 0; the words
- * must live until then.  Not under stream capture.
+ * must live until then, also after GTP_ERR_LAUNCH (the small kernel may be
+ * queued).  Not under stream capture.
  *
  * Replaces sequence_log_probs_from_logits  src/graspo/core/graspo_loss.py:19-21
  * and the forward of F.cross_entropy in sft_cross_entropy_loss
