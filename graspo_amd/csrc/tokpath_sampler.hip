@@ -2224,14 +2224,18 @@ bool spread_can(int64_t B, int64_t V, const gtp_sampler_params* p) {
 extern "C" size_t gtp_sample_spread_workspace_bytes(int64_t B, int64_t V,
                                                     const gtp_sampler_params* params) {
   if (!params || !spread_can(B, V, params)) return 0;
-  return spread::ws_bytes(B, spread::slices(B));
+  const int64_t R = spread::pass_rows(B);
+  return spread::ws_bytes(R, spread::slices(R), V);
 }
 
 // Where the spread kernels are the faster ones (us, both measured, the other
 // kernel first):
 // - Against the row-wise kernel always: fp16 [2, 151936] 134 / 29, fp16
 //   [256, 248320] 236 / 176, fp32 plain [16, 248320] 258 / 37, [256, 248320]
-//   335 / 218, bf16 [*, 50257] unaligned likewise.
+//   335 / 218, bf16 [*, 50257] unaligned likewise, and so large
+//   batches and small vocabularies (the row-wise kernel's LDS leaves one
+//   workgroup on a CU): fp16 [1024, 64] 133 /
+//   70, [16384, 256] 2089 / 1041, [4096, 151936] 3207 / 1748.
 // - Against the fp32 top-p kernel (two reads by one workgroup per row) up to
 //   96 rows: [8, 151936] 71 / 30, [48, 151936] 80 / 49, [96, 248320] 114 /
 //   103; [160, 151936] 83 / 104.
@@ -2278,7 +2282,7 @@ extern "C" int gtp_sample_rows_spread(const void* logits, int dtype, int64_t B, 
   if (rc != GTP_OK) return rc;
   if (B == 0) return GTP_OK;
   if (!spread_can(B, V, params)) return GTP_ERR_UNSUPPORTED;
-  if (!workspace || workspace_bytes < spread::ws_bytes(B, spread::slices(B)))
+  if (!workspace || workspace_bytes < gtp_sample_spread_workspace_bytes(B, V, params))
     return GTP_ERR_INVALID_ARGUMENT;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   switch (dtype) {

@@ -48,6 +48,7 @@ constexpr int kList = 8192;           // tokens of a row's two lists together
 constexpr int kSlice = 4096;          // tokens of a list from one slice
 constexpr int kSub = 256;             // parts of a list's bins
 constexpr int kSel = 2048;            // tokens of the part that is ranked
+constexpr int kRows = 4096;           // rows of one pass; more take several
 constexpr float kMMax = 32768.0f;     // |m| below this: step 3's pre-test margin
 constexpr int kG = 4;                 // groups of 8 tokens per thread and trip
 
@@ -70,16 +71,30 @@ struct Ws {
   SumPart* sum;
   u64* wbin;       // [B][S][kNB]
   uint32_t* cbin;  // [B][S][kNB]
-  u64* list;       // [B][2][kList] rank keys
+  u64* list;       // [B][cap] rank keys: the cut's list, then the draw's
+  int cap;
 };
 
+// Tokens of a row's two lists together.
+inline int list_cap(int64_t V) { return (int)(2 * V < kList ? 2 * V : kList); }
+
+// The workspace grows with the rows of a pass and not with the call's: at
+// most 300 MB (6 KB of bins per slice and up to 64 KB of lists per row), where
+// one pass over any batch took 9 GB at 65535 rows whatever V.  Passes of 1024
+// rows took 5 to 9% longer at 4096 rows and more (fp16 [4096, 151936] 1748 us
+// in one pass, 1913 in four).
 __host__ __device__ inline size_t align256(size_t n) { return (n + 255) / 256 * 256; }
-inline size_t ws_bytes(int64_t B, int S) {
+inline size_t ws_bytes(int64_t B, int S, int64_t V) {
   const size_t r = (size_t)B, rs = r * (size_t)S;
   return align256(r * sizeof(RowCtr)) + align256(rs * sizeof(MaxPart)) +
-         align256(rs * sizeof(SumPart)) + rs * kNB * 12 + r * 2 * kList * 8;
+         align256(rs * sizeof(SumPart)) + rs * kNB * 12 + align256(r * list_cap(V) * 8);
 }
-inline Ws ws_of(void* p, int64_t B, int S) {
+// Rows of a pass: as many passes as needed, of equal size.
+inline int64_t pass_rows(int64_t B) {
+  const int64_t passes = (B + kRows - 1) / kRows;
+  return (B + passes - 1) / passes;
+}
+inline Ws ws_of(void* p, int64_t B, int S, int64_t V) {
   unsigned char* q = reinterpret_cast<unsigned char*>(p);
   const size_t r = (size_t)B, rs = r * (size_t)S;
   auto take = [&](size_t n) {
@@ -93,7 +108,8 @@ inline Ws ws_of(void* p, int64_t B, int S) {
   w.sum = reinterpret_cast<SumPart*>(take(rs * sizeof(SumPart)));
   w.wbin = reinterpret_cast<u64*>(take(rs * kNB * 8));
   w.cbin = reinterpret_cast<uint32_t*>(take(rs * kNB * 4));
-  w.list = reinterpret_cast<u64*>(take(r * 2 * kList * 8));
+  w.cap = list_cap(V);
+  w.list = reinterpret_cast<u64*>(take(r * w.cap * 8));
   return w;
 }
 
@@ -508,7 +524,7 @@ __device__ __forceinline__ bool plan_row(const SamplerArgs& a, const Ws& ws, int
     p.before[l] = some ? sm.pre_c[p.lo[l]] : 0u;
     p.n[l] = some ? sm.pre_c[p.hi[l] + 1] - p.before[l] : 0u;
   }
-  return p.n[0] + p.n[1] <= (uint32_t)kList;
+  return p.n[0] + p.n[1] <= (uint32_t)ws.cap;
 }
 
 // The token of the list at sm.key[at0] (n tokens of bins [lo, hi], `base`
@@ -668,19 +684,17 @@ __device__ __forceinline__ bool pick_row(const SamplerArgs& a, const Ws& ws, int
                    : 0u;
   }
   __syncthreads();
+  u64* list = ws.list + b * ws.cap;
 #pragma unroll
   for (int l = 0; l < 2; ++l)
-    for (uint32_t i = tid; i < min(sm.n[l], (uint32_t)kSlice) && sm.at[l] + i < (uint32_t)kList; i += kB3)
-      put(ws.list + (b * 2 + l) * kList + sm.at[l] + i, sm.slice[l][i]);
+    for (uint32_t i = tid; i < min(sm.n[l], (uint32_t)kSlice) && sm.at[l] + i < p.n[l]; i += kB3)
+      put(list + (l ? p.n[0] : 0u) + sm.at[l] + i, sm.slice[l][i]);
   if (!arrive_last(&ws.ctr[b].pick, S)) return true;
   bool whole = true;
 #pragma unroll
   for (int l = 0; l < 2; ++l) whole = whole && take(&ws.ctr[b].len[l]) == p.n[l];
   if (!whole) return false;
-#pragma unroll
-  for (int l = 0; l < 2; ++l)
-    for (uint32_t i = tid; i < p.n[l]; i += kB3)
-      sm.key[(l ? p.n[0] : 0u) + i] = take(ws.list + (b * 2 + l) * kList + i);
+  for (uint32_t i = tid; i < p.n[0] + p.n[1]; i += kB3) sm.key[i] = take(list + i);
   __syncthreads();
   // the cut, then the draw
   u64 Wk = p.W;
@@ -734,24 +748,49 @@ inline int pick_slices(int64_t B) {
   return (int)(want < 1 ? 1 : want > kMaxS ? kMaxS : want);
 }
 
+// The call's rows from b0 on.
+template <typename T>
+SamplerArgs rows_from(SamplerArgs a, int64_t b0) {
+  a.logits = reinterpret_cast<const T*>(a.logits) + b0 * a.row_stride;
+  if (a.hist) a.hist += b0 * a.hist_stride;
+  if (a.mask) a.mask += b0 * a.mask_stride;
+  a.uniforms += b0;
+  if (a.finished) a.finished += b0;
+  a.out_ids += b0;
+  if (a.out_lp) a.out_lp += b0;
+  if (a.out_slp) a.out_slp += b0;
+  if (a.out_kept) a.out_kept += b0;
+  if (a.out_tv) a.out_tv += b0;
+  if (a.out_tid) a.out_tid += b0;
+  if (a.out_status) a.out_status += b0;
+  return a;
+}
+
+// Passes of pass_rows(B) rows over one workspace, each three launches.  They
+// follow one another on the stream, and each clears its own counters.
 template <typename T, bool kExtra>
-int launch_as(const SamplerArgs& a, int64_t B, void* workspace, hipStream_t s) {
-  const int S = slices(B), S3 = pick_slices(B);
-  const Ws ws = ws_of(workspace, B, S);
-  const dim3 grid((unsigned)S, (unsigned)B), grid3((unsigned)S3, (unsigned)B);
-  // the timing hook spans the three launches
+int launch_as(const SamplerArgs& call, int64_t B, void* workspace, hipStream_t s) {
+  const int64_t R = pass_rows(B);
+  const int S = slices(R), S3 = pick_slices(R);
+  const Ws ws = ws_of(workspace, R, S, call.V);
+  // the timing hook spans all launches
   const LaunchEvents e = g_next_launch_events;
   const bool timed = e.start && e.stop;
   g_next_launch_events = LaunchEvents{nullptr, nullptr};
-  if (timed)
-    hipExtLaunchKernelGGL((spread_max_kernel<T, kExtra>), grid, dim3(kT), 0, s, e.start, nullptr, 0, a, ws, S);
-  else
-    hipLaunchKernelGGL((spread_max_kernel<T, kExtra>), grid, dim3(kT), 0, s, a, ws, S);
-  hipLaunchKernelGGL((spread_weights_kernel<T, kExtra>), grid, dim3(kT), 0, s, a, ws, S);
-  if (timed)
-    hipExtLaunchKernelGGL(spread_pick_kernel<T>, grid3, dim3(kB3), 0, s, nullptr, e.stop, 0, a, ws, S3, S);
-  else
-    hipLaunchKernelGGL(spread_pick_kernel<T>, grid3, dim3(kB3), 0, s, a, ws, S3, S);
+  for (int64_t b0 = 0; b0 < B; b0 += R) {
+    const SamplerArgs a = rows_from<T>(call, b0);
+    const unsigned rows = (unsigned)(B - b0 < R ? B - b0 : R);
+    const dim3 grid((unsigned)S, rows), grid3((unsigned)S3, rows);
+    if (timed && b0 == 0)
+      hipExtLaunchKernelGGL((spread_max_kernel<T, kExtra>), grid, dim3(kT), 0, s, e.start, nullptr, 0, a, ws, S);
+    else
+      hipLaunchKernelGGL((spread_max_kernel<T, kExtra>), grid, dim3(kT), 0, s, a, ws, S);
+    hipLaunchKernelGGL((spread_weights_kernel<T, kExtra>), grid, dim3(kT), 0, s, a, ws, S);
+    if (timed && b0 + R >= B)
+      hipExtLaunchKernelGGL(spread_pick_kernel<T>, grid3, dim3(kB3), 0, s, nullptr, e.stop, 0, a, ws, S3, S);
+    else
+      hipLaunchKernelGGL(spread_pick_kernel<T>, grid3, dim3(kB3), 0, s, a, ws, S3, S);
+  }
   return hipGetLastError() == hipSuccess ? GTP_OK : GTP_ERR_LAUNCH;
 }
 

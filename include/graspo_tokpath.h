@@ -186,7 +186,8 @@ int gtp_sample_route(int dtype, int64_t B, int64_t V, int aligned, int64_t hist_
  * three launches, any dtype, alignment and vocabulary; the same arguments and
  * bit-exact results.  The workspace is required
  * (gtp_sample_spread_workspace_bytes, 0 for a call it does not take), 256-byte
- * aligned, no contents carried between calls.
+ * aligned, no contents carried between calls; at most 300 MB, for large
+ * batches run in passes over it.
  * gtp_sample_spread_wins tells whether it is the faster one for a call
  * (aligned, hist_len and has_mask as in gtp_sample_route); the torch op asks
  * it.

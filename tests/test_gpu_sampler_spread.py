@@ -178,6 +178,37 @@ def test_repeated_calls_on_a_used_workspace_and_in_a_graph():
             assert torch.equal(getattr(out, f), getattr(eager, f)), f
 
 
+@pytest_gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("B,V", [(4097, 40), (8200, 301)])
+def test_passes_over_large_batches(dtype, B, V):
+    """Two and three passes over one workspace, the last one shorter: every
+    per-row argument and output moves along."""
+    g = torch.Generator().manual_seed(B)
+    x = (torch.randn(B, V + 3, generator=g) * 3).to(dtype)[:, 1 : V + 1]
+    hist = torch.randint(-1, V, (B, 9), generator=g, dtype=torch.int32)
+    hist[B - 1, 4] = V
+    fin = (torch.rand(B, generator=g) < 0.1).to(torch.uint8)
+    for kw in (dict(temperature=0.8), dict(temperature=0.7, top_p=0.9, repetition_penalty=1.2,
+                                           history=hist, allow_mask=_mask(B, V, g, 0.6),
+                                           finished=fin, pad_token_id=5)):
+        _check(f"passes {dtype} [{B}, {V}] {sorted(kw)}", x, uniforms=_u(B, g), **kw)
+
+
+def test_workspace_is_bounded():
+    """The workspace depends on the rows of a pass and on V, not on the batch."""
+    L = _lib()
+    p = _capi.SamplerParams(0.7, 0, 0.9, 1.0)
+
+    def size(B, V):
+        return L.gtp_sample_spread_workspace_bytes(B, V, ctypes.byref(p))
+
+    for V in (1, 64, 4096, 151936, 1 << 18):
+        most = max(size(B, V) for B in (1, 32, 512, 4096, 4097, 8192, 65535))
+        assert most <= 4096 * (16 * min(V, 4096) + 512 * 12 + 128) + 4096, V
+    assert size(65535, 64) < 32 << 20 and size(65535, 151936) < 300 << 20
+
+
 def test_spread_query_on_the_host():
     """Which calls the spread kernels take; arguments refused before launch."""
     L = _lib()
