@@ -8,6 +8,7 @@
 // (torch.cuda.current_stream().cuda_stream), so work orders with the
 // caller's other torch work exactly as the reference's ATen ops did.
 #include <ATen/ATen.h>
+#include <ATen/EmptyTensor.h>
 #include <torch/library.h>
 
 #include <map>
@@ -79,19 +80,6 @@ bool rows_aligned(const at::Tensor& logits) {
          ((uint64_t)(row_stride_of(logits) * logits.element_size()) & 15u) == 0;
 }
 
-// The next n elements of a byte tensor's storage as a tensor of their own, on
-// 16 bytes.  One allocation for a call's seven outputs instead of seven: a
-// greedy call of one row, whose kernel takes 7 us, 12.3 -> 9.9 us.
-at::Tensor part_of(const at::Tensor& pool, int64_t& at_byte, int64_t n, at::ScalarType type) {
-  at::Tensor t = at::detail::make_tensor<c10::TensorImpl>(
-      c10::Storage(pool.storage()), pool.key_set(), at::scalarTypeToTypeMeta(type));
-  const int64_t size = (int64_t)at::elementSize(type);
-  t.unsafeGetTensorImpl()->set_storage_offset(at_byte / size);
-  t.unsafeGetTensorImpl()->set_sizes_contiguous({n});
-  at_byte += (n * size + 15) / 16 * 16;
-  return t;
-}
-
 using SampleOut =
     std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor, at::Tensor, at::Tensor, at::Tensor>;
 
@@ -150,16 +138,18 @@ SampleOut sample(const at::Tensor& logits, double temperature, int64_t top_k, do
     fin = static_cast<const uint8_t*>(f.data_ptr());
   }
   auto opt = logits.options();
-  const int64_t word = (B * 4 + 15) / 16 * 16;
-  const at::Tensor pool = at::empty({(B * 8 + 15) / 16 * 16 + 6 * word}, opt.dtype(at::kByte));
-  int64_t at_byte = 0;
-  at::Tensor ids = part_of(pool, at_byte, B, at::kLong);
-  at::Tensor lp = part_of(pool, at_byte, B, at::kFloat);
-  at::Tensor slp = part_of(pool, at_byte, B, at::kFloat);
-  at::Tensor kept = part_of(pool, at_byte, B, at::kInt);
-  at::Tensor tv = part_of(pool, at_byte, B, at::kFloat);
-  at::Tensor tid = part_of(pool, at_byte, B, at::kInt);
-  at::Tensor st = part_of(pool, at_byte, B, at::kInt);
+  // Each output has a storage of its own (it can be saved, resized or handed
+  // to another stream by itself).  Six of the seven come from the allocator
+  // directly: a greedy call of one row, whose kernel takes 7 us, takes 12.1 us
+  // with seven at::empty, 10.9 this way (9.4 as parts of one allocation).
+  const at::Tensor ids = at::empty({B}, opt.dtype(at::kLong));
+  c10::Allocator* const alloc = ids.storage().allocator();
+  const c10::DeviceGuard guard(logits.device());
+  auto output = [&](at::ScalarType type) {
+    return at::Tensor(at::detail::empty_generic({B}, alloc, ids.key_set(), type, c10::nullopt));
+  };
+  const at::Tensor lp = output(at::kFloat), slp = output(at::kFloat), kept = output(at::kInt),
+                   tv = output(at::kFloat), tid = output(at::kInt), st = output(at::kInt);
   gtp_sampler_params p;
   p.temperature = (float)temperature;
   p.top_k = (int32_t)top_k;

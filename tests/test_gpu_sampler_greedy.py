@@ -102,8 +102,8 @@ def test_greedy_special_rows(workspace, V):
 @pytest.mark.parametrize("B", [0, 1, 3, 5])
 @pytest.mark.parametrize("inference", [False, True])
 def test_outputs_are_tensors_of_their_own(B, inference):
-    """The seven outputs share an allocation, not memory: each is contiguous,
-    keeps its dtype, and writing one in place leaves the others."""
+    """Each of the seven outputs is contiguous, keeps its dtype, and writing
+    one in place leaves the others."""
     from graspo_amd import ops
 
     x = torch.randn(B, 4096, device=DEV)
@@ -122,3 +122,32 @@ def test_outputs_are_tensors_of_their_own(B, inference):
                 if j > i:
                     assert torch.equal(o, before[j])
     assert not any(t.requires_grad for t in out)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kw", [dict(temperature=0.0), dict(temperature=0.8, top_k=20),
+                                dict(temperature=1.0, top_p=0.9)])
+def test_outputs_have_storages_of_their_own(kw):
+    """They can be saved together and resized, and each is freed on its own."""
+    import io
+
+    from graspo_amd import ops
+
+    out = ops.sample(torch.randn(3, 4096, device=DEV), **kw)
+    assert len({t.untyped_storage().data_ptr() for t in out}) == 7
+    for t in out:
+        assert t.storage_offset() == 0
+        assert t.untyped_storage().nbytes() == t.numel() * t.element_size()
+    f = io.BytesIO()
+    torch.save(tuple(out), f)
+    f.seek(0)
+    for a, b in zip(torch.load(f, weights_only=True), out):
+        assert torch.equal(a.cpu(), b.cpu())
+    before = [t.clone() for t in out]
+    out.ids.resize_(64).fill_(-1)
+    out.kept.resize_(64).fill_(-1)
+    for t, b in list(zip(out, before))[1:3] + list(zip(out, before))[4:]:
+        assert torch.equal(t, b)
+    with torch.cuda.device(DEV):
+        side = torch.cuda.Stream()
+        out.logprob.record_stream(side)
