@@ -23,14 +23,17 @@ class _SFTCrossEntropy(torch.autograd.Function):
                                 mean=True)
         if out.bad_target:  # F.cross_entropy rejects a label outside [0, V)
             raise RuntimeError("sft_cross_entropy_loss: a label is outside [0, vocab_size)")
-        ctx.save_for_backward(logits, labels, out.logprob, out.count)
+        # a copy of the targets (behind the rows, 8 bytes each): a loader may
+        # refill its labels before the backward
+        targets = labels[:, 1:].clone() if ctx.needs_input_grad[0] else None
+        ctx.save_for_backward(logits, targets, out.logprob, out.count)
         ctx.ignore_index = ignore_index
         return out.mean_loss
 
     @staticmethod
     def backward(ctx, grad_loss):
-        logits, labels, lp, count = ctx.saved_tensors
-        grad = ops.token_logprob_backward(logits, labels[:, 1:], lp, grad_loss, mean_count=count,
+        logits, targets, lp, count = ctx.saved_tensors
+        grad = ops.token_logprob_backward(logits, targets, lp, grad_loss, mean_count=count,
                                           ignore_index=ctx.ignore_index)
         return grad, None, None
 

@@ -95,6 +95,19 @@ def test_sft_shifted_rows(B, S, V, dtype):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.int64, torch.int32])
+def test_sft_labels_refilled_before_the_backward(dtype):
+    g = torch.Generator().manual_seed(3)
+    x = torch.randn(2, 9, 500, generator=g).to(DEV).requires_grad_(True)
+    labels = torch.randint(0, 500, (2, 9), generator=g).to(DEV, dtype)
+    (want,) = torch.autograd.grad(sft_cross_entropy_loss(x, labels), [x])
+    loss = sft_cross_entropy_loss(x, labels)
+    labels.fill_(-100)
+    (got,) = torch.autograd.grad(loss, [x])
+    assert torch.equal(got, want) and bool(want.any())
+
+
+@pytest.mark.gpu
 def test_sft_one_position_and_no_targets():
     x = torch.randn(2, 1, 64, device=DEV, requires_grad=True)
     loss = sft_cross_entropy_loss(x, torch.zeros(2, 1, dtype=torch.int64, device=DEV))
