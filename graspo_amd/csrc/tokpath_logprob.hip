@@ -481,10 +481,10 @@ __global__ __launch_bounds__(kLpBlock) void token_logprob_backward_kernel(
                             slices > 1 ? (int)(blockIdx.x - n * slices) : 0, slices);
 }
 
-// loss = -sum_n lp_n v_n / count, count = sum_n v_n, v_n = 1 unless row n is
-// ignored: F.cross_entropy's mean.  An ignored row is multiplied by 0, so a
-// non-finite logprob of it shows in the loss.  One workgroup: at most some
-// ten thousand rows, 4 bytes of logprob and one target each.
+// loss = -sum lp_n / count over the count rows that are not ignored:
+// F.cross_entropy's mean, which no value of an ignored row reaches (its
+// logprob, token 0's, may be NaN or -inf).  One workgroup: at most some ten
+// thousand rows, 4 bytes of logprob and one target each.
 __global__ __launch_bounds__(1024) void token_mean_kernel(TokenRows a, int64_t N,
                                                           const float* __restrict__ lp,
                                                           float* __restrict__ loss,
@@ -496,9 +496,9 @@ __global__ __launch_bounds__(1024) void token_mean_kernel(TokenRows a, int64_t N
   for (int64_t n = threadIdx.x; n < N; n += 1024) {
     int64_t b, s;
     a.at(n, b, s);
-    const bool v = !(a.has_ignore && a.target(b, s) == a.ignore);
-    sum += (double)(lp[n] * (v ? 1.0f : 0.0f));
-    c += v;
+    if (a.has_ignore && a.target(b, s) == a.ignore) continue;
+    sum += (double)lp[n];
+    ++c;
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {

@@ -108,6 +108,29 @@ def test_sft_labels_refilled_before_the_backward(dtype):
 
 
 @pytest.mark.gpu
+def test_sft_ignored_rows_of_any_value():
+    """A NaN in an ignored row, or token 0 at -inf there, does not reach the
+    loss or the gradient, as in F.cross_entropy."""
+    g = torch.Generator().manual_seed(4)
+    x = torch.randn(2, 7, 300, generator=g)
+    labels = torch.randint(0, 300, (2, 7), generator=g)
+    labels[0, 1:4] = -100  # the targets of positions 0..2
+    x[0, 0, 17] = float("nan")
+    x[0, 1, 0] = float("-inf")
+    x[0, 2] = float("-inf")
+    x[1, 6] = float("nan")  # the last position has no target
+    xd = x.to(DEV).requires_grad_(True)
+    loss = sft_cross_entropy_loss(xd, labels.to(DEV))
+    (grad,) = torch.autograd.grad(loss, [xd])
+    keep = labels[:, 1:].ne(-100)
+    ls = x[:, :-1].double().log_softmax(-1)
+    ref = F.nll_loss(ls[keep], labels[:, 1:][keep])
+    assert float(loss.detach()) == pytest.approx(float(ref), abs=LP_TOL)
+    assert bool((grad[:, :-1][~keep.to(DEV)] == 0).all()) and bool((grad[:, -1] == 0).all())
+    assert bool(grad.isfinite().all())
+
+
+@pytest.mark.gpu
 def test_sft_one_position_and_no_targets():
     x = torch.randn(2, 1, 64, device=DEV, requires_grad=True)
     loss = sft_cross_entropy_loss(x, torch.zeros(2, 1, dtype=torch.int64, device=DEV))
