@@ -61,6 +61,29 @@ def test_slices(N, V, dtype):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("N", [2, 2100])
+def test_entropy_where_the_first_infinities_come_late(N, dtype):
+    """Blocks before, at and after the first one that holds a -inf, in rows of
+    slices and of one workgroup: single logits, a tail and a whole step."""
+    V = 70001
+    g = torch.Generator().manual_seed(N)
+    x = (torch.randn(8, V, generator=g) * 3).to(dtype)
+    for r, at in enumerate((0, 1, 16384, 40000, V - 1)):
+        x[r, at] = -float("inf")
+    x[5, 33000:] = -float("inf")
+    x[6, 20000:60000] = -float("inf")
+    t = torch.full((8,), 7)
+    n = (N + 7) // 8
+    out = ops.token_logprob(x.to(DEV).repeat(n, 1)[:N], t.to(DEV).repeat(n)[:N], entropy=True)
+    rlp, rH = _ref(x, t)
+    for k in range(0, N, 8):
+        m = min(8, N - k)
+        assert float((out.logprob[k : k + m].cpu() - rlp[:m]).abs().max()) <= LP_TOL
+        assert float((out.entropy[k : k + m].cpu() - rH[:m]).abs().max()) <= LP_TOL
+
+
+@pytest.mark.gpu
 def test_non_finite_rows_in_slices():
     V = 151936
     x = torch.zeros(4, V, dtype=torch.bfloat16)
