@@ -14,6 +14,18 @@
 namespace gtp {
 
 constexpr int kNbBlock = 256;
+
+// Tells that the workgroup saw a value that is not a bf16 value; call with
+// every thread.  One look at the word per workgroup, which leaves it when it
+// is set: an atomic of every wave on the one word took longer than the pass
+// ([96, 151936] with such values throughout
+// 400 us more, now 30).
+__device__ __forceinline__ void report_inexact(uint32_t low, uint32_t* inexact) {
+  if (__syncthreads_or((int)low) && threadIdx.x == 0 &&
+      __hip_atomic_load(inexact, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u)
+    atomicOr(inexact, 1u);
+}
+
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 __global__ __launch_bounds__(kNbBlock) void narrow_bf16_vec_kernel(const u32x4* __restrict__ src,
@@ -42,7 +54,7 @@ __global__ __launch_bounds__(kNbBlock) void narrow_bf16_vec_kernel(const u32x4* 
       if (i < n4) __builtin_nontemporal_store(o, dst + i);
     }
   }
-  if (__ballot(low != 0u) && (threadIdx.x & (kWave - 1)) == 0) atomicOr(inexact, 1u);
+  report_inexact(low, inexact);
 }
 
 // any alignment and the elements past the last whole group of four
@@ -56,7 +68,7 @@ __global__ __launch_bounds__(kNbBlock) void narrow_bf16_scalar_kernel(
     low |= v & 0xFFFFu;
     dst[i] = (uint16_t)(v >> 16);
   }
-  if (__ballot(low != 0u) && (threadIdx.x & (kWave - 1)) == 0) atomicOr(inexact, 1u);
+  report_inexact(low, inexact);
 }
 
 }  // namespace gtp

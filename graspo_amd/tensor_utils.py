@@ -17,11 +17,30 @@ from torch.nn import functional as F  # noqa: N812
 from . import ops
 
 
+# From so many fp32 logits on, and from this vocabulary on, the
+# value-histogram kernel on a bf16 copy takes less time than the spread
+# kernels on the rows as they are, the copy's pass and host synchronisation
+# included.  Plain rows, us, spread / copy and histogram: [208, 65536] 104 /
+# 96, [96, 151936] 126 / 113, [64, 248320] 128 / 123, [256, 151936] 194 / 145,
+# [256, 248320] 281 / 190; below, [64, 151936] 101 / 107, [48, 248320] 118 /
+# 119, [128, 65536] 80 / 89; smaller vocabularies [1024, 32000] 190 / 197,
+# [2048, 16000] 230 / 295.  Rows that are not contiguous are gathered first:
+# [96, 248320] 164 / 156, [64, 248320] 123 / 137.
+_NARROW_FROM = 13_000_000
+_NARROW_STRIDED_FROM = 24_000_000
+_NARROW_VOCAB = 65536
+
+
 def _fp32_kernel_takes(logits: torch.Tensor, temperature: float, top_k: int,
                        top_p: float) -> bool:
-    """Whether an fp32 call without history or mask goes to the spread or the
-    fp32 top-p kernels, as the library's own routing decides."""
-    if ops.sample_spread(logits, temperature=temperature, top_k=top_k, top_p=top_p):
+    """Whether an fp32 call without history or mask is faster on its fp32
+    rows than on a bf16 copy: the fp32 top-p kernel's calls, and the spread
+    kernels' of fewer logits than above or whose copy would have unaligned
+    rows, for which there is no histogram kernel."""
+    least = _NARROW_FROM if logits.is_contiguous() else _NARROW_STRIDED_FROM
+    V = logits.shape[1]
+    if ((logits.numel() < least or V < _NARROW_VOCAB or V % 8 != 0)
+            and ops.sample_spread(logits, temperature=temperature, top_k=top_k, top_p=top_p)):
         return True
     route, _ = ops.sample_route(logits, temperature=temperature, top_k=top_k, top_p=top_p)
     return route == ops.ROUTE_TOPP32
@@ -31,12 +50,10 @@ def _bf16_when_exact(logits: torch.Tensor, temperature: float, top_k: int,
                      top_p: float = 1.0) -> torch.Tensor:
     """fp32 rows as their bf16 copy when every value is a bf16 value -- the
     reference's callers pass ``logits.float()`` of a bf16 model -- and the
-    call would otherwise take the row-wise kernel (sampling with a top-k above
-    128; the spread and the fp32 top-p kernels read the rows directly, which
-    is faster than the narrowing and its host synchronisation): the
-    value-histogram kernel takes bf16 rows only, and
-    the samples are the same because the float inputs are.  Costs one pass
-    over the rows and one host synchronisation."""
+    bf16 kernels are the faster ones with the copy: large batches without a
+    top-p cut, and calls that would take the row-wise kernel (sampling with a
+    top-k above 128).  The samples are the same because the float inputs are.
+    Costs one pass over the rows and one host synchronisation."""
     if (logits.dtype != torch.float32 or logits.dim() != 2 or not logits.is_cuda
             or not temperature > 0 or 1 <= top_k <= 128
             or _fp32_kernel_takes(logits, temperature, top_k, top_p)):
