@@ -439,10 +439,14 @@ __global__ __launch_bounds__(256) void lm_head_target_kernel(const uint16_t* __r
 
 // Folds the partial states of each token: 16 tokens per workgroup, 16
 // groups of threads each merging every 16th partial (a group reads 256
-// contiguous bytes per partial), then one merge in LDS.
+// contiguous bytes per partial), then one merge in LDS.  With one tile per
+// group, two of them (of one wave half) merge first, as the running state of
+// a group of two does: a token's result does not depend on how many tokens
+// there are (nor on the tiles per group that their number picks).  n_full:
+// the full vocabulary tiles then, 0 with groups of two.
 constexpr int kMergeTok = 16, kMergeGrp = 16;
 __global__ __launch_bounds__(256) void lm_head_merge_kernel(const float4* __restrict__ partial,
-                                                            int nsub, int64_t N,
+                                                            int nsub, int n_full, int64_t N,
                                                             const float* __restrict__ xt,
                                                             float* __restrict__ out_lp,
                                                             float* __restrict__ out_H,
@@ -453,10 +457,23 @@ __global__ __launch_bounds__(256) void lm_head_merge_kernel(const float4* __rest
   const int64_t n = (int64_t)blockIdx.x * kMergeTok + lt;
   Lse3 st{kNegInf, 0.0f, 0.0f};
   if (n < N) {
+    auto at = [&](int q) {
+      const float4 v = partial[(int64_t)q * N + n];
+      return Lse3{v.x, v.y, v.z};
+    };
+    if (n_full == 0) {
 #pragma unroll 4
-    for (int p = g; p < nsub; p += kMergeGrp) {
-      const float4 v = partial[(int64_t)p * N + n];
-      st = merge_states(st, Lse3{v.x, v.y, v.z});
+      for (int p = g; p < nsub; p += kMergeGrp) st = merge_states(st, at(p));
+    } else {
+#pragma unroll 4
+      for (int p = g; p < nsub; p += kMergeGrp) {
+        const int half = p & 1, tile = p - half;  // tiles `tile` and `tile` + 1
+        const int q = 2 * min(tile, n_full) + half;
+        Lse3 a = at(q);
+        const Lse3 b = at(tile + 1 < n_full ? q + 2 : q);
+        if (tile + 1 < n_full) a = merge_states(a, b);
+        st = merge_states(st, a);
+      }
     }
   }
   red[g][lt][0] = st.m;
@@ -570,8 +587,9 @@ int lm_head_run(const uint16_t* hidden, int64_t N, int64_t K, int64_t hidden_str
                      xt);
   hipLaunchKernelGGL(lmh::lm_head_merge_kernel,
                      dim3((unsigned)((N + lmh::kMergeTok - 1) / lmh::kMergeTok)), dim3(256), 0, s,
-                     a.partial, 2 * p.n_vg + (p.tail ? 2 : 0), N, xt, out_logprob, out_entropy,
-                     out_lse, out_status);
+                     a.partial, 2 * ((p.n_vfull + 1) / 2) + (p.tail ? 2 : 0),
+                     p.tiles == 1 ? p.n_vfull : 0, N, xt, out_logprob, out_entropy, out_lse,
+                     out_status);
   return hipGetLastError() == hipSuccess ? GTP_OK : GTP_ERR_LAUNCH;
 }
 }  // namespace
