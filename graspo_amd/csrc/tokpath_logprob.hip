@@ -55,24 +55,6 @@ __device__ __forceinline__ int64_t row_head(const T* row, int64_t V) {
   return up % sizeof(T) ? V : min((int64_t)(up / sizeof(T)), V);
 }
 
-// Block-wide (m, s, t) in wave 0's lanes.  `red` holds one state per wave.
-// The reduction is a kernel's tail once per row or slice: with shuffles and
-// pairwise merges the kernel of 61 rows of 151936 bf16 logits took 13.0 us,
-// this way 11.6.
-__device__ __forceinline__ Lse3 block_lse3_wave0(Lse3 v, float (*red)[3]) {
-  v = wave_lse3_max(v);
-  const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
-  if (lane == 0) {
-    red[wid][0] = v.m;
-    red[wid][1] = v.s;
-    red[wid][2] = v.t;
-  }
-  __syncthreads();
-  const int w = lane & (kLpBlock / kWave - 1);
-  const bool in = lane < kLpBlock / kWave;
-  return wave_lse3_max(in ? Lse3{red[w][0], red[w][1], red[w][2]} : Lse3{kNegInf, 0.0f, 0.0f});
-}
-
 // Calls f(i) for this thread's share of the elements outside
 // [head, head + body).
 template <typename F>
@@ -122,26 +104,91 @@ __device__ __forceinline__ void lp_fold_block(Lse3& st, const float (&x)[NG][E],
   }
 }
 
-// This thread's share of slice k of a row [0, V).
+// A row's sum is cut in chunks of whole steps of the stream, `per` steps each
+// and at most kMaxChunks of them, by its vocabulary alone: a chunk's state is
+// the merge of its four waves' and a row's is the merge of its chunks',
+// whichever workgroups take them.  So a row has the same bits scored alone, in
+// a small batch (where its chunks go to several workgroups) and in a large
+// one.
+constexpr int kMaxChunks = 32;
+constexpr int kLpStep = kLpBlock * kLpVecs;  // vectors
+struct Chunks {
+  int n, per;
+};
+template <typename T>
+Chunks chunks_of(int64_t V) {
+  const int64_t steps = max((int64_t)1, (V / Vec<T>::kE + kLpStep - 1) / kLpStep);
+  const int64_t per = (steps + kMaxChunks - 1) / kMaxChunks;
+  return {(int)((steps + per - 1) / per), (int)per};
+}
+
+// The four waves' states of a chunk, as wave_lse3_max merges lanes.
+__device__ __forceinline__ Lse3 merge_waves(const float (*red)[kMaxChunks][3], int c) {
+  constexpr int kW = kLpBlock / kWave;
+  float m = red[0][c][0];
+#pragma unroll
+  for (int w = 1; w < kW; ++w) m = fmaxf(m, red[w][c][0]);
+  float s = 0.0f, t = 0.0f;
+#pragma unroll
+  for (int w = 0; w < kW; ++w) {
+    const float wm = red[w][c][0], ws = red[w][c][1];
+    const float dl = wm == m ? 0.0f : fmaxf((wm - m) * kLog2e, -256.0f);
+    const float f = __builtin_amdgcn_exp2f(dl);
+    s += ws * f;
+    t += f * __builtin_fmaf(dl, ws, red[w][c][2]);
+  }
+  return {m, s, t};
+}
+
+// Chunks [c0, c1) of a row [0, V): lane l of wave 0 gets chunk c0 + l's state
+// (the lanes past them an empty one).  Every thread calls; `red` is the
+// workgroup's.  A wave reduces its chunk as soon as it has folded it, on DPP:
+// a call of bf16 [8192, 151936], ten chunks a row, 381 us with one reduction
+// per row, 384 with ten (375 with the shorter prefetch past the stream's end).
 template <typename T, bool kEntropy>
-__device__ __forceinline__ Lse3 lp_thread_state(const T* __restrict__ row, int64_t V, int k,
-                                                int slices) {
+__device__ __forceinline__ Lse3 chunk_states(const T* __restrict__ row, int64_t V, Chunks ch,
+                                             int c0, int c1, float (*red)[kMaxChunks][3]) {
   constexpr int E = Vec<T>::kE;
-  Lse3 st{kNegInf, 0.0f, 0.0f};
+  const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
   const int64_t head = row_head(row, V);
   const int64_t nvec = (V - head) / E;
-  const Slice sl = slice_of<E>(nvec, k, slices);
+  const int64_t v0 = min((int64_t)c0 * ch.per * kLpStep, nvec);
+  const int64_t v1 = min((int64_t)c1 * ch.per * kLpStep, nvec);
+  const bool partial = (v1 - v0) % kLpStep != 0;
+  const Lse3 empty{kNegInf, 0.0f, 0.0f};
+  Lse3 st = empty, held = empty;
+  int c = 0, left = ch.per;
   bool clamp = false;
-  const bool partial = (sl.v1 - sl.v0) % (kLpBlock * kLpVecs) != 0;
+  auto close = [&]() __attribute__((always_inline)) {
+    if constexpr (kEntropy)
+      st = wave_lse3_max(st);
+    else
+      wave_lse2(st.m, st.s);
+    if (lane == c) held = st;
+    st = empty;
+    left = ch.per;
+    ++c;
+  };
   stream_vectors<T, kLpBlock, kLpVecs, true>(
-      row + head, sl.v0, sl.v1, [&](float(&x)[kLpVecs][E], int64_t vbase, bool last) {
-        if (last) mask_tail<kLpVecs, E, kLpBlock>(x, vbase, sl.v1);
+      row + head, v0, v1, [&](float(&x)[kLpVecs][E], int64_t vbase, bool last) {
+        if (left == 0) close();
+        --left;
+        if (last) mask_tail<kLpVecs, E, kLpBlock>(x, vbase, v1);
         lp_fold_block<kEntropy, kLpVecs, E>(st, x, clamp, last && partial);
       });
-  // the row's ends go to its last slice
-  if (sl.last)
+  // the row's ends go to its last chunk
+  if (c1 == ch.n) {
+    if (c < ch.n - 1 - c0) close();
     for_edges(V, head, nvec * E, [&](int64_t i) { lse_fold_one(st, Elem<T>::get(row, i)); });
-  return st;
+  }
+  close();
+  if (lane < c1 - c0) {
+    red[wid][lane][0] = held.m;
+    red[wid][lane][1] = held.s;
+    red[wid][lane][2] = held.t;
+  }
+  __syncthreads();
+  return lane < c1 - c0 ? merge_waves(red, lane) : empty;
 }
 
 __device__ __forceinline__ int64_t load_target(const void* targets, int t64, int64_t n) {
@@ -229,16 +276,16 @@ __global__ __launch_bounds__(kVerdictBlock) void token_targets_kernel(
   __hip_atomic_store(verdict + blockIdx.x, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// slices == 1: one workgroup per row.  Otherwise workgroup (row, slice)
-// publishes its (m, s, t), and the last of the row's workgroups to arrive
-// merges them in order (so the result does not depend on which one that is).
-// A second launch for the merge took 4 us after the 12 of 61 rows.
+// slices == 1: one workgroup per row.  Otherwise workgroup (row, slice) takes
+// its share of the row's chunks and publishes their (m, s, t), and the last of
+// the row's workgroups to arrive merges them.  A second launch for the merge
+// took 4 us after the 12 of 61 rows.
 template <typename T, bool kEntropy>
 __global__ __launch_bounds__(kLpBlock) void token_logprob_kernel(TokenRows a, TokenOut out,
-                                                                 int slices,
+                                                                 Chunks ch, int slices,
                                                                  uint32_t* __restrict__ ctr,
                                                                  float* __restrict__ partial) {
-  __shared__ float red[kLpBlock / kWave][3];
+  __shared__ float red[kLpBlock / kWave][kMaxChunks][3];
   // (rows in slices are few: one dimension)
   const int64_t n = slices > 1 ? blockIdx.x / (uint32_t)slices : flat_workgroup();
   if (n >= a.rows()) return;
@@ -250,30 +297,34 @@ __global__ __launch_bounds__(kLpBlock) void token_logprob_kernel(TokenRows a, To
   const bool ok = tgt >= 0 && tgt < a.V;
   float xt = 0.0f;
   if (threadIdx.x == 0 && ok) xt = Elem<T>::get(row, tgt);
-  Lse3 st = block_lse3_wave0(lp_thread_state<T, kEntropy>(row, a.V, k, slices), red);
+  const int c0 = k * ch.n / slices, c1 = (k + 1) * ch.n / slices;
+  Lse3 st = chunk_states<T, kEntropy>(row, a.V, ch, c0, c1, red);
   if (threadIdx.x >= kWave) return;
+  const int lane = threadIdx.x;
   if (slices > 1) {
     // No release operation: gfx950's agent-scope stores write through to
     // where the other XCDs' agent-scope loads see them, and vmcnt(0) waits
     // for their completion before the arrival (a release fence would write
     // the whole L2 back).
-    float* p = partial + (n * slices + k) * 3;
-    if (threadIdx.x < 3)
-      __hip_atomic_store(p + threadIdx.x, threadIdx.x == 0 ? st.m : threadIdx.x == 1 ? st.s : st.t,
-                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    float* p = partial + n * ch.n * 3;  // [3][chunks]
+    if (lane < c1 - c0) {
+      __hip_atomic_store(p + c0 + lane, st.m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(p + ch.n + c0 + lane, st.s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(p + 2 * ch.n + c0 + lane, st.t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     uint32_t arrived = 0;
-    if (threadIdx.x == 0)
+    if (lane == 0)
       arrived = __hip_atomic_fetch_add(ctr + n, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (__builtin_amdgcn_readfirstlane((int)arrived) != slices - 1) return;
     asm volatile("" ::: "memory");
-    // lane k holds slice k (at most kMaxSlices = 32 of them)
-    p = partial + (n * slices + min((int)threadIdx.x, slices - 1)) * 3;
+    p += min(lane, ch.n - 1);
     const float m = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const float sm = __hip_atomic_load(p + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const float t = __hip_atomic_load(p + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    st = wave_lse3_max((int)threadIdx.x < slices ? Lse3{m, sm, t} : Lse3{kNegInf, 0.0f, 0.0f});
+    const float sm = __hip_atomic_load(p + ch.n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const float t = __hip_atomic_load(p + 2 * ch.n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    st = lane < ch.n ? Lse3{m, sm, t} : Lse3{kNegInf, 0.0f, 0.0f};
   }
+  st = wave_lse3_max(st);
   if (threadIdx.x == 0) out.put(n, st, xt, ok);
 }
 
@@ -281,12 +332,15 @@ __global__ __launch_bounds__(kLpBlock) void token_logprob_kernel(TokenRows a, To
 template <typename T>
 __global__ __launch_bounds__(kLpBlock) void lse_partial_kernel(
     const T* __restrict__ logits, int64_t Vc, int64_t row_stride, int64_t col_offset,
-    const void* __restrict__ targets, int t64, float* __restrict__ state, int accumulate) {
-  __shared__ float red[kLpBlock / kWave][3];
+    const void* __restrict__ targets, int t64, float* __restrict__ state, int accumulate,
+    Chunks ch) {
+  __shared__ float red[kLpBlock / kWave][kMaxChunks][3];
   const int64_t n = blockIdx.x;
   const T* row = logits + n * row_stride;
   const int64_t tgt = targets ? load_target(targets, t64, n) - col_offset : -1;
-  Lse3 st = block_lse3_wave0(lp_thread_state<T, true>(row, Vc, 0, 1), red);
+  Lse3 st = chunk_states<T, true>(row, Vc, ch, 0, ch.n, red);
+  if (threadIdx.x >= kWave) return;
+  st = wave_lse3_max(st);
   if (threadIdx.x == 0) {
     float* sp = state + n * 4;
     float xt = __builtin_nanf("");
@@ -589,24 +643,25 @@ __global__ __launch_bounds__(kLpBlock) void logprob_backward_split_kernel(
 using namespace gtp;
 
 namespace {
-constexpr int kMaxRowSlices = 32;
-
-// Workgroups per row: eight resident workgroups on every CU when there are
-// fewer rows than that, each with about one full step of its stream (32 KB)
-// or more; one per row otherwise.  bf16 [61, 151936] takes 11.6 us in ten
-// slices and 15.7 us in one workgroup per row; from 8 x 256 rows on the chip
-// is full without them ([8192, 151936] runs at 6.5 TB/s of the 7.0 that a
-// read-only pass reaches).
-int row_slices(int dtype, int64_t N, int64_t V) {
-  const int64_t nvec = V / (dtype == GTP_DTYPE_F32 ? 4 : 8);
-  const int64_t step = kLpBlock * kLpVecs;
-  const int64_t want = (8 * device_cus() + N - 1) / N;
-  return (int)max((int64_t)1, min(min(want, (int64_t)kMaxRowSlices), (nvec + step - 1) / step));
+// Chunks of a row's sum, and the slices of the gradient.
+Chunks row_chunks(int dtype, int64_t V) {
+  return dtype == GTP_DTYPE_F32 ? chunks_of<float>(V) : chunks_of<uint16_t>(V);
 }
 
-// Workspace: the rows' arrival counters, then 3 floats per slice.
-size_t row_slices_bytes(int64_t N, int slices) {
-  return slices > 1 ? (size_t)N * 4 + (size_t)(N * slices) * 12 : 0;
+// Workgroups per row: eight resident workgroups on every CU when there are
+// fewer rows than that, each with a chunk or more (mostly one full step of
+// its stream, 32 KB); one per row otherwise.  bf16 [61, 151936] takes 11.6 us
+// in ten slices and 15.7 us in one workgroup per row; from 8 x 256 rows on the
+// chip is full without them ([8192, 151936] runs at 6.5 TB/s of the 7.0 that a
+// read-only pass reaches).
+int row_slices(int dtype, int64_t N, int64_t V) {
+  const int64_t want = (8 * device_cus() + N - 1) / N;
+  return (int)max((int64_t)1, min(want, (int64_t)row_chunks(dtype, V).n));
+}
+
+// Workspace: the rows' arrival counters, then 3 floats per chunk.
+size_t row_slices_bytes(int64_t N, int slices, int chunks) {
+  return slices > 1 ? (size_t)N * 4 + (size_t)(N * chunks) * 12 : 0;
 }
 
 // The look at the targets: a few thousand per workgroup; the words of
@@ -622,12 +677,13 @@ void targets_launch(const TokenRows& a, int64_t N, uint32_t* ctr, int n_ctr, con
 template <typename T>
 void token_logprob_launch(const TokenRows& a, const TokenOut& out, int64_t N, int slices,
                           uint32_t* ctr, hipStream_t s) {
+  const Chunks ch = chunks_of<T>(a.V);
   const dim3 grid = flat_grid(N * slices), block(kLpBlock);
   float* partial = reinterpret_cast<float*>(ctr + (slices > 1 ? N : 0));
   if (out.H)
-    launch_timed(token_logprob_kernel<T, true>, grid, block, s, a, out, slices, ctr, partial);
+    launch_timed(token_logprob_kernel<T, true>, grid, block, s, a, out, ch, slices, ctr, partial);
   else
-    launch_timed(token_logprob_kernel<T, false>, grid, block, s, a, out, slices, ctr, partial);
+    launch_timed(token_logprob_kernel<T, false>, grid, block, s, a, out, ch, slices, ctr, partial);
 }
 
 // GTP_OK and the device form of `r`, with sequences that follow one another
@@ -660,7 +716,7 @@ void join_rows(TokenRows& a, int64_t St) {
 
 extern "C" size_t gtp_token_logprob_workspace_bytes(int dtype, int64_t N, int64_t V) {
   if (N <= 0 || V <= 0 || N > 0x3FFFFFFll) return 0;
-  return row_slices_bytes(N, row_slices(dtype, N, V));
+  return row_slices_bytes(N, row_slices(dtype, N, V), row_chunks(dtype, V).n);
 }
 
 extern "C" int gtp_token_logprob_rows(const gtp_token_rows* rows, float* out_logprob,
@@ -678,7 +734,9 @@ extern "C" int gtp_token_logprob_rows(const gtp_token_rows* rows, float* out_log
   join_rows(a, a.S);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   int slices = row_slices(rows->dtype, N, a.V);
-  if (!workspace || workspace_bytes < row_slices_bytes(N, slices)) slices = 1;
+  if (!workspace ||
+      workspace_bytes < row_slices_bytes(N, slices, row_chunks(rows->dtype, a.V).n))
+    slices = 1;
   uint32_t* ctr = reinterpret_cast<uint32_t*>(workspace);
   if (slices > 1 || verdict)
     targets_launch(a, N, ctr, slices > 1 ? (int)N : 0, nullptr, nullptr, verdict, s);
@@ -891,17 +949,17 @@ extern "C" int gtp_lse_partial_rows(const void* logits, int dtype, int64_t N, in
     case GTP_DTYPE_BF16:
       hipLaunchKernelGGL(lse_partial_kernel<uint16_t>, grid, block, 0, s,
                          reinterpret_cast<const uint16_t*>(logits), Vc, row_stride, col_offset,
-                         targets, targets_int64, state, accumulate);
+                         targets, targets_int64, state, accumulate, chunks_of<uint16_t>(Vc));
       break;
     case GTP_DTYPE_F16:
       hipLaunchKernelGGL(lse_partial_kernel<_Float16>, grid, block, 0, s,
                          reinterpret_cast<const _Float16*>(logits), Vc, row_stride, col_offset,
-                         targets, targets_int64, state, accumulate);
+                         targets, targets_int64, state, accumulate, chunks_of<_Float16>(Vc));
       break;
     case GTP_DTYPE_F32:
       hipLaunchKernelGGL(lse_partial_kernel<float>, grid, block, 0, s,
                          reinterpret_cast<const float*>(logits), Vc, row_stride, col_offset,
-                         targets, targets_int64, state, accumulate);
+                         targets, targets_int64, state, accumulate, chunks_of<float>(Vc));
       break;
     default:
       return GTP_ERR_INVALID_ARGUMENT;
