@@ -8,9 +8,12 @@
 // call.  Each row is cut into S slices; every thread folds its tokens into
 // (m, s) and its best (y, id), and the last of the row's workgroups to arrive
 // merges the slices.  Rows may start at any element.  The slices and their
-// threads' shares are the split kernel's, so a slice of up to four vectors per
-// thread gives the same log-sum-exp to the bit: the logprob of a row that is
-// nearly one-hot, ln(1 + a little), magnifies a unit of the sum.
+// threads' shares are the split kernel's, so in 16-bit types a slice within
+// that kernel's pilot (four vectors per thread, three in fp16) gives the same
+// log-sum-exp to the bit: the logprob of a row that is nearly one-hot, ln(1 +
+// a little), magnifies a unit of the sum.  (Past its pilot the split kernel's
+// waves share a slice out as they go, and its sum varies from call to call;
+// this kernel's never does.)
 //
 // Bound by the latency of a launch, one trip to memory and the arrival on
 // small batches, by the stream on large ones.  bf16 [1, 151936], the split

@@ -122,3 +122,30 @@ def sample_small_workspace(logits: torch.Tensor, **kw):
     assert rc == 0, rc
     torch.cuda.synchronize()
     return out.cpu()
+
+
+def sample_rows(logits: torch.Tensor, *, history=None, finished=None, uniforms=None, **kw):
+    """gtp_sample_rows with the workspace that it asks for: the kernel that
+    gtp_sample_route names, where the torch op may take another.  Arguments as
+    ops.sample's, on the logits' device; returns (outputs on the CPU as a dict
+    of the SampleOutput fields, route)."""
+    L = lib()
+    if history is not None:
+        history = history.to(torch.int32).contiguous() if history.numel() else None
+    if finished is not None:
+        finished = finished.to(torch.uint8)
+    mask = kw.pop("allow_mask", None)
+    args, p, B = sample_args(logits, history=history, finished=finished, uniforms=uniforms,
+                             allow_mask=None if mask is None else mask.contiguous(), **kw)
+    dt, V = DTYPE[logits.dtype], logits.shape[1]
+    n = L.gtp_sample_workspace_bytes(dt, B, V, ctypes.byref(p))
+    ws = torch.zeros(max(n, 256), dtype=torch.uint8, device=logits.device)
+    out = SampleBuffers(B, logits.device)
+    assert L.gtp_sample_rows(*args, *out.out_args(), ws.data_ptr() if n else None, n,
+                             stream_handle()) == 0
+    torch.cuda.synchronize()
+    es = logits.element_size()
+    r, _ = route(L, dt, B, V, T=p.temperature, k=p.top_k, P=p.top_p, rho=p.repetition_penalty,
+                 hist_len=0 if history is None else history.shape[1], mask=mask is not None,
+                 aligned=logits.data_ptr() % 16 == 0 and logits.stride(0) * es % 16 == 0)
+    return out.cpu(), r

@@ -12,6 +12,7 @@ import torch
 from graspo_amd import ops
 from graspo_amd import workloads as W
 from oracle import oracle as O
+from tests import _capi
 from tests._util import oracle_sample
 
 pytestmark = pytest.mark.gpu
@@ -22,12 +23,36 @@ def _to(t, dev):
     return None if t is None else t.to(dev)
 
 
-def gpu_sample(logits, **kw):
+def gpu_sample(logits, route=None, **kw):
+    """ops.sample's outputs on the CPU.  Where the op takes the spread kernels,
+    the kernel that gtp_sample_rows takes for the same call runs too and must
+    give the same bits (the logprobs within TOL).  ``route``: that kernel's."""
     dev = torch.device("cuda:0")
     kw = {k: (_to(v, dev) if isinstance(v, torch.Tensor) else v) for k, v in kw.items()}
-    out = ops.sample(logits.to(dev), **kw)
+    logits = logits.to(dev)
+    out = ops.sample(logits, **kw)
     torch.cuda.synchronize()
-    return ops.SampleOutput(*[t.cpu() for t in out])
+    out = ops.SampleOutput(*[t.cpu() for t in out])
+    hist = kw.get("history")
+    spread = ops.sample_spread(
+        logits, temperature=kw["temperature"], top_k=kw.get("top_k", 0),
+        top_p=kw.get("top_p", 1.0), repetition_penalty=kw.get("repetition_penalty", 1.0),
+        hist_len=0 if hist is None else hist.shape[1], has_mask=kw.get("allow_mask") is not None)
+    if spread or route is not None:
+        direct, took = _capi.sample_rows(logits, **kw)
+        assert route is None or took == route, (took, route)
+        ok = out.status == 0
+        for f in ("status", "ids", "kept", "thresh_id", "thresh_value"):
+            a, b = getattr(out, f), direct[f]
+            if f not in ("status", "ids"):
+                a, b = a[ok], b[ok]
+            if f == "thresh_value":
+                a, b = a.view(torch.int32), b.view(torch.int32)
+            assert torch.equal(a, b), (f, took)
+        for f in ("logprob", "sampled_logprob"):
+            a, b = getattr(out, f)[ok], direct[f][ok]
+            assert torch.allclose(a, b, rtol=0.0, atol=TOL, equal_nan=True), (f, took)
+    return out
 
 
 def assert_parity(g, ref, what=""):

@@ -7,13 +7,16 @@ its rank among equal values, in id order), penalised and out-of-range
 tokens kept one by one, the rows that leave the histogram for the row-wise
 path (too many out-of-range tokens, an exact tie between a penalised token
 and a value bin, crowded value segments), vocabularies with a tail,
-extreme temperatures and the per-row statuses."""
+extreme temperatures and the per-row statuses.  Every case runs
+gtp_sample_rows (below 65536 tokens, and without a top-p cut, that is the
+value-histogram kernel), and the torch op beside it, which takes the spread
+kernels for up to 16 rows without top-k."""
 
 import numpy as np
 import pytest
 import torch
 
-from graspo_amd import workloads as W
+from graspo_amd import ops, workloads as W
 from tests._util import oracle_sample
 from tests.test_gpu_sampler import assert_parity, gpu_sample
 
@@ -48,7 +51,8 @@ def test_dense_value_bins(top_p, top_k):
     for T in (0.7, 1.0):
         kw = dict(temperature=T, top_k=top_k, top_p=top_p, uniforms=u)
         print("dense", top_p, top_k, T, flush=True)
-        assert_parity(gpu_sample(x, **kw), oracle_sample(x, **kw), f"p{top_p} k{top_k} T{T}")
+        route = ops.ROUTE_HIST if top_k or top_p == 1.0 else None
+        assert_parity(gpu_sample(x, route, **kw), oracle_sample(x, **kw), f"p{top_p} k{top_k} T{T}")
 
 
 @pytest.mark.parametrize("rho", [1.3, 0.7])
@@ -104,7 +108,7 @@ def test_vocab_tail(V):
     u = _edge_uniforms(6, g)
     kw = dict(temperature=0.8, top_p=0.95, repetition_penalty=1.2, history=hist, uniforms=u)
     dev = torch.device("cuda:0")
-    out = gpu_sample(full.to(dev)[:, :V], **kw)
+    out = gpu_sample(full.to(dev)[:, :V], ops.ROUTE_HIST if V < 65536 else None, **kw)
     assert_parity(out, oracle_sample(x.contiguous(), **kw), f"V{V}")
 
 
@@ -115,7 +119,8 @@ def test_extreme_temperature(T):
     x = x.to(torch.bfloat16)
     u = _edge_uniforms(6, g)
     kw = dict(temperature=T, top_p=0.9, uniforms=u)
-    assert_parity(gpu_sample(x, **kw), oracle_sample(x, **kw), f"T{T}")
+    route = ops.ROUTE_HIST if T <= 1024 else ops.ROUTE_ROWWISE
+    assert_parity(gpu_sample(x, route, **kw), oracle_sample(x, **kw), f"T{T}")
 
 
 def test_status_rows_bf16():
@@ -137,4 +142,4 @@ def test_status_rows_bf16():
     fin[7] = True
     kw = dict(temperature=1.0, top_p=0.9, repetition_penalty=1.2, history=hist,
               allow_mask=W.pack_mask(bits), uniforms=u, finished=fin, pad_token_id=-5)
-    assert_parity(gpu_sample(x, **kw), oracle_sample(x, **kw))
+    assert_parity(gpu_sample(x, ops.ROUTE_HIST, **kw), oracle_sample(x, **kw))

@@ -61,8 +61,13 @@ def _check(what, x, general=True, **kw):
         ok = ref.status == 0
         assert np.array_equal(got["thresh_value"].numpy()[ok].view(np.int32),
                               ref.thresh_value[ok].view(np.int32)), (what, name)
-        assert np.abs(got["logprob"].numpy()[ok] - ref.logprob[ok]).max(initial=0) <= 1e-3
-        assert np.abs(got["sampled_logprob"].numpy()[ok] - ref.sampled_logprob[ok]).max(initial=0) <= 1e-3
+        # fp32 sums of up to 2^18 terms (a few 1e-6 relative), a logarithm and a
+        # difference below 32 (2e-6 each); the exponents' rounding, 1e-6 a term
+        for f in ("logprob", "sampled_logprob"):
+            a, b = got[f].numpy()[ok], getattr(ref, f)[ok]
+            fin = np.isfinite(b)
+            assert np.array_equal(a[~fin], b[~fin], equal_nan=True), (what, name, f)
+            assert np.abs(a[fin] - b[fin]).max(initial=0) <= 2e-5, (what, name, f)
 
 
 def _u(B, g):

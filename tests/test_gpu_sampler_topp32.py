@@ -36,7 +36,9 @@ def _u(B, g):
 def _check(x, what, **kw):
     print("topp32:", what, tuple(x.shape), {k: v for k, v in kw.items()
                                             if not isinstance(v, torch.Tensor)}, flush=True)
-    g = gpu_sample(x, **kw)
+    # gtp_sample_rows takes the fp32 top-p kernel for these rows, whichever
+    # kernels the torch op takes for so few
+    g = gpu_sample(x, route=ops.ROUTE_TOPP32 if x.shape[1] >= 65536 else None, **kw)
     ref = oracle_sample(x, **kw)
     assert_parity(g, ref, what)
     return g, ref
