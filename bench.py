@@ -72,7 +72,7 @@ HBM_PEAK_GBS = 8000.0
 PREWARM_S = 0.3  # seconds of untimed steps before the warm-up steps
 REPO = os.path.dirname(os.path.abspath(__file__))
 SAMPLER_KERNEL = "sampler_split_kernel<bf16>"
-LOGPROB_KERNEL = "logprob_entropy_kernel<bf16>"
+LOGPROB_KERNEL = "token_logprob_kernel<bf16>"
 BACKWARD_KERNEL = "logprob_backward_kernel<bf16>"
 TRAFFIC_FILE = os.path.join(REPO, "profiles", "hbm_traffic_large_vocab.md")
 if REPO not in sys.path:

@@ -27,8 +27,8 @@ def _token_rows(logits: torch.Tensor) -> torch.Tensor | None:
 def _rows_logprob_entropy(logits: torch.Tensor, output_ids: torch.Tensor, entropy: bool = True):
     """(logprob, entropy) over the last dim of ``logits`` [..., V] (entropy
     empty unless asked for); a target outside [0, V) raises ``RuntimeError``,
-    as the reference's ``gather`` rejects such an index (one wait for the
-    kernel).  Views whose leading dims fit no [B, S, V] without a copy are
+    as the reference's ``gather`` rejects such an index (one wait, for a look
+    at the targets that runs ahead of the rows).  Views whose leading dims fit no [B, S, V] without a copy are
     walked per slice."""
     V = logits.shape[-1]
     lead = logits.shape[:-1]

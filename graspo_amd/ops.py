@@ -2,8 +2,9 @@
 
 Each function validates nothing beyond what the native op checks, enqueues
 the HIP kernels on the caller's current stream and returns device tensors;
-none of them synchronises the host except ``token_logprob``, whose callers
-raise on a bad target.
+none of them waits for the GPU except ``token_logprob`` and
+``TargetsVerdict.wait``, which wait for a look at the targets, so that a
+caller can raise on a bad one.
 """
 
 from __future__ import annotations
@@ -149,9 +150,11 @@ def token_logprob(logits: torch.Tensor, targets: torch.Tensor, *, ignore_index: 
                   entropy: bool = False, mean: bool = False) -> TokenLogprob:
     """log_softmax(logits)[targets] over [S, V] or [B, S, V] ``logits`` (unit
     column stride, read in place) and ``targets`` of their leading shape, one
-    HBM read.  ``entropy`` adds the rows' softmax entropies, ``mean`` the mean
-    cross-entropy over the targets that are not ``ignore_index`` (an ignored
-    row's logprob is token 0's).  Waits for a look at the targets, which runs
+    HBM read.  A row's result has the same bits whatever rows are passed with
+    it (rows at the same alignment).  ``entropy`` adds the rows' softmax
+    entropies, ``mean`` the mean cross-entropy over the targets that are not
+    ``ignore_index`` (an ignored row's logprob is token 0's; no value of such
+    a row reaches the mean).  Waits for a look at the targets, which runs
     ahead of the rows, to say whether one is bad."""
     return TokenLogprob(*load().token_logprob(logits, _targets(targets), ignore_index, entropy,
                                               mean, _stream(logits)))

@@ -284,7 +284,8 @@ typedef struct gtp_token_rows {
  * token 0's.  Few rows are cut into slices for several workgroups each, whose
  * partial states go through a workspace of gtp_token_logprob_workspace_bytes
  * (B * S rows) bytes, 16-byte aligned, no contents carried between calls;
- * without one (or when that is 0) each row is one workgroup's.
+ * without one (or when that is 0) each row is one workgroup's.  A row's
+ * result has the same bits either way, and whatever rows are passed with it.
  *
  * verdict, when given, is GTP_VERDICT_WORDS words of host memory that the
  * device can write (pinned), each GTP_VERDICT_PENDING before the call: a
@@ -325,7 +326,8 @@ int gtp_targets_verdict(const void* targets, int targets_int64, int64_t N, int64
 int gtp_stream_capturing(void* stream);
 
 /* gtp_token_mean_loss -- *loss = -sum logprob / *count over the rows that are
- * not ignored (NaN when there is none), *count their number. */
+ * not ignored (NaN when there is none), *count their number.  No value of an
+ * ignored row reaches the loss. */
 int gtp_token_mean_loss(const gtp_token_rows* rows, const float* logprob, float* loss,
                         int64_t* count, void* stream);
 
