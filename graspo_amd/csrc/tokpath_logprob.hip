@@ -650,9 +650,9 @@ Chunks row_chunks(int dtype, int64_t V) {
 
 // Workgroups per row: eight resident workgroups on every CU when there are
 // fewer rows than that, each with a chunk or more (mostly one full step of
-// its stream, 32 KB); one per row otherwise.  bf16 [61, 151936] takes 11.6 us
-// in ten slices and 15.7 us in one workgroup per row; from 8 x 256 rows on the
-// chip is full without them ([8192, 151936] runs at 6.5 TB/s of the 7.0 that a
+// its stream, 32 KB); one per row otherwise.  bf16 [61, 151936] takes 10.5 us
+// in ten slices and 16.4 us in one workgroup per row; from 8 x 256 rows on the
+// chip is full without them ([8192, 248320] runs at 6.8 TB/s of the 7.0 that a
 // read-only pass reaches).
 int row_slices(int dtype, int64_t N, int64_t V) {
   const int64_t want = (8 * device_cus() + N - 1) / N;
