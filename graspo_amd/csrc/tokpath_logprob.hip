@@ -324,7 +324,7 @@ __global__ __launch_bounds__(kLpBlock) void token_logprob_kernel(TokenRows a, To
     const float t = __hip_atomic_load(p + 2 * ch.n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     st = lane < ch.n ? Lse3{m, sm, t} : Lse3{kNegInf, 0.0f, 0.0f};
   }
-  st = wave_lse3_max(st);
+  if (ch.n > 1) st = wave_lse3_max(st);
   if (threadIdx.x == 0) out.put(n, st, xt, ok);
 }
 
@@ -340,7 +340,7 @@ __global__ __launch_bounds__(kLpBlock) void lse_partial_kernel(
   const int64_t tgt = targets ? load_target(targets, t64, n) - col_offset : -1;
   Lse3 st = chunk_states<T, true>(row, Vc, ch, 0, ch.n, red);
   if (threadIdx.x >= kWave) return;
-  st = wave_lse3_max(st);
+  if (ch.n > 1) st = wave_lse3_max(st);
   if (threadIdx.x == 0) {
     float* sp = state + n * 4;
     float xt = __builtin_nanf("");
