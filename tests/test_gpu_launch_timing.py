@@ -79,16 +79,21 @@ def test_hook_spans_a_row_that_takes_the_row_wise_path():
     times = {}
     for name, xx in (("plain", x), ("handed_over", xh)):
         ops.sample(xx, **kw)  # warm
-        k0, k1 = _events()
-        o0, o1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-        ops.time_next_launch(k0, k1)
-        o0.record()
-        out = ops.sample(xx, **kw)
-        o1.record()
-        torch.cuda.synchronize()
-        times[name] = (k0.elapsed_time(k1), o0.elapsed_time(o1))
-        assert bool((out.status == 0).all())
+        hooked, around = [], []
+        for _ in range(9):
+            k0, k1 = _events()
+            o0, o1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            ops.time_next_launch(k0, k1)
+            o0.record()
+            out = ops.sample(xx, **kw)
+            o1.record()
+            torch.cuda.synchronize()
+            hooked.append(k0.elapsed_time(k1))
+            around.append(o0.elapsed_time(o1))
+            assert bool((out.status == 0).all())
+            assert 0.0 < hooked[-1] <= around[-1]
+        # the shortest of each: the host can be held up between the outer events
+        times[name] = (min(hooked), min(around))
     print("top-p call (hooked, around):", times, flush=True)
     (t0, a0), (t1, a1) = times["plain"], times["handed_over"]
-    assert 0.0 < t0 <= a0 and 0.0 < t1 <= a1
     assert t1 - t0 > 0.5 * (a1 - a0) > 0.0
