@@ -1,10 +1,12 @@
 // torch_ops.cpp -- thin PyTorch-ROCm binding of the C ABI (host-only C++).
 //
-// Registers torch.ops.graspo_tokpath.{sample, sample_route, logprob_entropy, logprob_backward, graspo_loss_*, lse_partial,
-// lse_finalize, decode_update, to_bf16_exact, logprob_backward_split, time_next_launch,
-// lm_head_logprob, lm_head_logprob_save, softmax_grad_bf16}.  Each op validates its tensors (TORCH_CHECK surfaces as a
-// Python RuntimeError), allocates the outputs on the logits' device, and
-// enqueues the HIP kernels on the stream handle passed in from Python
+// Registers torch.ops.graspo_tokpath.{sample, sample_route, sample_spread,
+// logprob_entropy, token_logprob, token_logprob_backward, verdict_begin,
+// verdict_end, logprob_backward, graspo_loss_*, lse_partial, lse_finalize,
+// decode_update, to_bf16_exact, logprob_backward_split, time_next_launch,
+// lm_head_logprob, lm_head_logprob_save, softmax_grad_bf16}.  Each op validates
+// its tensors (TORCH_CHECK surfaces as a Python RuntimeError), allocates the
+// outputs on the logits' device, and enqueues the HIP kernels on the stream handle passed in from Python
 // (torch.cuda.current_stream().cuda_stream), so work orders with the
 // caller's other torch work exactly as the reference's ATen ops did.
 #include <ATen/ATen.h>

@@ -572,7 +572,9 @@ int gtp_f32_to_bf16_exact(const float* src, int64_t n, uint16_t* dst,
  * when its kernel's dispatch begins and stop_event when it ends
  * (hipExtLaunchKernelGGL; each of these calls is one launch), so the two HIP
  * events bracket the call's kernel, without the idle time of event packets
- * recorded around it.
+ * recorded around it.  Around gtp_sample_rows_spread they bracket all its
+ * launches; gtp_token_logprob_rows, gtp_token_logprob_backward, the lm_head and
+ * the softmax gradient calls record their one large kernel.
  * Both are hipEvent_t created by the caller (with timing).  The hook is per
  * thread and used once; the benchmark is its caller.
  */
