@@ -13,10 +13,12 @@
 #include <ATen/EmptyTensor.h>
 #include <torch/library.h>
 
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <tuple>
 #include <utility>
+#include <vector>
 
 #include "graspo_tokpath.h"
 
@@ -62,18 +64,21 @@ void check_same_device(const at::Tensor& a, const at::Tensor& b, const char* nam
 
 // Sampler workspace, one per (device, stream): zero-filled when allocated (the
 // library keeps it reusable from call to call), grown when a call needs more.
-// Calls on one stream are ordered, so they can share it.
+// Calls on one stream are ordered, so they can share it.  One that has been
+// outgrown is kept, for a captured graph may hold its address; a new one is
+// at least twice as large, so all of them together stay below twice the last.
 void* sampler_workspace(const at::Tensor& like, size_t bytes, int64_t stream) {
   if (bytes == 0) return nullptr;
   static std::mutex mu;
-  static std::map<std::pair<int, int64_t>, at::Tensor> cache;
+  static std::map<std::pair<int, int64_t>, std::vector<at::Tensor>> cache;
   std::lock_guard<std::mutex> lock(mu);
-  at::Tensor& ws = cache[{(int)like.get_device(), stream}];
-  if (!ws.defined() || (size_t)ws.numel() < bytes) {
-    const int64_t n = (int64_t)((bytes + 4095) / 4096 * 4096);
-    ws = at::zeros({n}, like.options().dtype(at::kByte));
+  std::vector<at::Tensor>& all = cache[{(int)like.get_device(), stream}];
+  if (all.empty() || (size_t)all.back().numel() < bytes) {
+    const size_t least = all.empty() ? 0 : 2 * (size_t)all.back().numel();
+    const int64_t n = (int64_t)((std::max(bytes, least) + 4095) / 4096 * 4096);
+    all.push_back(at::zeros({n}, like.options().dtype(at::kByte)));
   }
-  return ws.data_ptr();
+  return all.back().data_ptr();
 }
 
 // 16-byte aligned logits and row stride

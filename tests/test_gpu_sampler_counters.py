@@ -1,12 +1,14 @@
 """Calls of different row counts on one workspace: the arrival counters of
 more than 4096 split rows (fp32 above 131072 tokens) reach into what is slot
-data for a smaller call."""
+data for a smaller call; a captured call keeps its workspace when the stream's
+is outgrown."""
 
 import ctypes
 
 import pytest
 import torch
 
+from graspo_amd import ops
 from tests import _capi
 
 DEV = torch.device("cuda:0")
@@ -46,3 +48,33 @@ def test_counters_beyond_the_fixed_region(how):
                 assert float((v - first[f][:rows]).abs().max()) <= 1e-5
             else:
                 assert torch.equal(v, first[f][:rows]), f
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("offset", [0, 1])
+def test_captured_call_after_the_workspace_has_grown(offset):
+    """Greedy rows, aligned and not: the workspace that a graph was captured
+    with stays its own when a larger call on the stream has outgrown it."""
+    V = 151936
+    stream = torch.cuda.Stream()
+    g = torch.Generator(device=DEV).manual_seed(2)
+    x = torch.randn(1, V + 8, generator=g, device=DEV).bfloat16()[:, offset : offset + V]
+    big = torch.randn(130, V + 8, generator=g, device=DEV).bfloat16()[:, offset : offset + V]
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        ops.sample(x, temperature=0.0)
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=stream):
+        out = ops.sample(x, temperature=0.0)
+    with torch.cuda.stream(stream):
+        ids = ops.sample(big, temperature=0.0).ids
+        mine = [torch.full((1 << 15,), 7, dtype=torch.uint8, device=DEV) for _ in range(64)]
+    torch.cuda.synchronize()
+    assert torch.equal(ids, big.argmax(1))
+    for k in range(3):
+        x.copy_(torch.randn(1, V, generator=g, device=DEV))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert int(out.ids) == int(x.argmax(1)), k
+        assert all(bool((t == 7).all()) for t in mine)
